@@ -649,6 +649,10 @@ extern "C" int ti_tern_gemm(ti_ctx* c, float* out, long out_stride, const uint8_
     TI_REQUIRE(out && codes && scales && act && xsum, "ti_tern_gemm: null buffer");
     TI_REQUIRE(N > 0 && K > 0 && K % 64 == 0 && B > 0 && out_stride >= N, "ti_tern_gemm: bad shape (N=%d K=%d B=%d)", N, K, B);
     TI_REQUIRE(al16(codes) && al16(act), "ti_tern_gemm: codes and act must be 16-byte aligned");
+    // up to 4 rows stay on the row kernels (bit-identical to gemv_tern, and one launch where K has a
+    // batched instance); from 5 on they would take a launch per row: 191 us at 2048 x 6144 x 50
+    if (B > 4 && ti_tern_gemm_mfma_ok(N, K, B))
+        return ti_tern_gemm_mfma(c, act, xsum, K, B, 1, &codes, &scales, &out, &out_stride, &N);
     // batches of 4 share each code unpack (lib.rs gemm_tern_b4); a tail runs as B=2/1
     int done = 0;
     while (done < B) {

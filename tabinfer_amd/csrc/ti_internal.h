@@ -117,6 +117,9 @@ bool ti_tern_swiglu_ok(int K);
 int ti_tern_gemv_swiglu(ti_ctx* c, const ti_tern_swiglu* sw, float* out, const uint8_t* codes, const float* scales, int N,
                         int K);
 bool ti_tern_norm_ok(int K);
+bool ti_tern_gemm_mfma_ok(int N, int K, int B);
+int ti_tern_gemm_mfma(ti_ctx* c, const int8_t* act, const int32_t* xsum, int K, int B, int nmat, const uint8_t* const* codes,
+                      const float* const* scales, float* const* outs, const long* strides, const int* Ns);
 int ti_tern_gemv_multi_norm(ti_ctx* c, const ti_tern_norm* nq, int K, int nmat, const uint8_t* const* codes,
                             const float* const* scales, float* const* outs, const int* Ns);
 bool ti_tgemm_ok(int T, int K);
