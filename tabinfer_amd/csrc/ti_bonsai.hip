@@ -16,6 +16,7 @@
 // the step embeds hist[P], writes KV row P, and (with logits) puts the argmax in hist[P+1]
 // and advances P.
 #include "ti_internal.h"
+#include "ti_bonsai_batch.h"
 #include <math.h>
 #include <string.h>
 #include <stdio.h>
@@ -628,6 +629,14 @@ struct ti_bonsai {
     float* rope;          // [max_ctx][head_dim]: cos then sin of each position (ops.rs rope_table)
     float* rope_cur;      // the row of the device position, kept in step with dpos
     uint32_t* trace = nullptr;
+    // the T-token path: rows [batch][width] of the buffers above, one allocation
+    int batch = 0;        // tokens of one batch, at most
+    long rowsplits = 0;   // attention partials
+    struct {
+        float *x, *q, *k, *v, *qrot, *o, *g, *u, *d, *scales, *po, *pml;
+        uint32_t* act;
+        int32_t* xsum;
+    } b;
     std::vector<void*> allocs;
 };
 
@@ -743,6 +752,26 @@ extern "C" int ti_bonsai_create(ti_ctx* c, const ti_bonsai_config* cfg, ti_bonsa
     if (!rc) rc = bmk(m, (void**)&m->dpos, 4);
     if (!rc) rc = bmk(m, (void**)&m->rope, (size_t)C.max_ctx * hd * 4);
     if (!rc) rc = bmk(m, (void**)&m->rope_cur, (size_t)hd * 4);
+    if (!rc) {
+        m->batch = C.max_ctx < TI_BB_TOKENS ? C.max_ctx : TI_BB_TOKENS;
+        m->rowsplits = (long)m->batch * C.n_heads * TI_BB_SPLITS;
+        if (m->rowsplits > TI_BB_ROWSPLITS) m->rowsplits = TI_BB_ROWSPLITS;
+        const size_t B = m->batch;
+        struct { void** p; size_t words; } part[] = {
+            {(void**)&m->b.x, B * H}, {(void**)&m->b.q, B * nq}, {(void**)&m->b.k, B * nkv}, {(void**)&m->b.v, B * nkv},
+            {(void**)&m->b.qrot, B * nq}, {(void**)&m->b.o, B * H}, {(void**)&m->b.g, B * I}, {(void**)&m->b.u, B * I},
+            {(void**)&m->b.d, B * H}, {(void**)&m->b.scales, 4 * B}, {(void**)&m->b.po, (size_t)m->rowsplits * hd},
+            {(void**)&m->b.pml, (size_t)m->rowsplits * 2}, {(void**)&m->b.act, B * widest / 4},
+            {(void**)&m->b.xsum, B * widest / 64}};
+        size_t words = 0;
+        for (auto& f : part) words += (f.words + 63) / 64 * 64;      // 256-byte aligned parts
+        char* slab = nullptr;
+        rc = bmk(m, (void**)&slab, words * 4);
+        for (auto& f : part) {
+            *f.p = slab;
+            slab += (f.words + 63) / 64 * 256;
+        }
+    }
     if (!rc) {
         // ops.rs:79-90 in f32 with the platform's powf / cosf / sinf, the functions Rust's
         // f32::powf and sin_cos call on Linux
@@ -936,6 +965,32 @@ static int bn_norm_quant(ti_ctx* c, float* x, const float* add, const float* add
     return TI_OK;
 }
 
+// The final norm of x + down / down_scale, lm_head, the logits and their argmax: into
+// hist[P + 1] at the device position P, which advances.
+static int bonsai_logits(ti_ctx* c, ti_bonsai* m, float* x, const float* down, const float* down_scale) {
+    const ti_bonsai_config& C = m->cfg;
+    const int H = C.hidden, hd = C.head_dim;
+    float* sa = m->scales;
+    int rc;
+    if ((rc = bn_norm_quant(c, x, down, down_scale, m->final_norm, C.rms_eps, H, m->xn, m->act, m->xsum, sa))) return rc;
+    if (m->trace) {
+        uint32_t* fin = bslot(m, C.layers, 0);
+        // x_final, xn_final, its codes and scale after the last layer
+        k_bn_copy_u32<<<8, 256, 0, c->stream>>>(reinterpret_cast<const uint32_t*>(x), fin, H);
+        k_bn_copy_u32<<<8, 256, 0, c->stream>>>(reinterpret_cast<const uint32_t*>(m->xn), fin + H, H);
+        k_bn_copy_u32<<<8, 256, 0, c->stream>>>(reinterpret_cast<const uint32_t*>(m->act), fin + 2 * H, H / 4);
+        k_bn_copy_u32<<<1, 64, 0, c->stream>>>(reinterpret_cast<const uint32_t*>(sa), fin + 2 * H + H / 4, 1);
+        TI_LAUNCHED("k_bn_copy_u32 (trace)");
+    }
+    if ((rc = ti_tern_gemv(c, m->lraw, m->lm.codes, m->lm.scales, m->act, m->xsum, C.vocab, H))) return rc;
+    k_bn_logits<<<BN_AMAX_PARTS, 256, 0, c->stream>>>(m->lraw, sa, C.vocab, m->logits, m->amax_v, m->amax_i);
+    TI_LAUNCHED("k_bn_logits");
+    k_bn_argmax<<<1, BN_AMAX_PARTS, 0, c->stream>>>(m->amax_v, m->amax_i, BN_AMAX_PARTS, m->hist, m->dpos, C.max_ctx, m->rope,
+                                                    m->rope_cur, hd);
+    TI_LAUNCHED("k_bn_argmax");
+    return TI_OK;
+}
+
 // One token at the device position P (model.rs:349-501): with logits, the argmax goes to
 // hist[P + 1]; P advances either way.
 static int bonsai_step(ti_ctx* c, ti_bonsai* m, bool want_logits) {
@@ -1062,23 +1117,7 @@ static int bonsai_step(ti_ctx* c, ti_bonsai* m, bool want_logits) {
         TI_LAUNCHED("k_bn_advance");
         return TI_OK;
     }
-    RC(bn_norm_quant(c, m->x, m->draw, sd, m->final_norm, C.rms_eps, H, m->xn, m->act, m->xsum, sa));
-    if (m->trace) {
-        uint32_t* fin = bslot(m, C.layers, 0);
-        // x_final, xn_final, its codes and scale after the last layer
-        k_bn_copy_u32<<<8, 256, 0, c->stream>>>(reinterpret_cast<const uint32_t*>(m->x), fin, H);
-        k_bn_copy_u32<<<8, 256, 0, c->stream>>>(reinterpret_cast<const uint32_t*>(m->xn), fin + H, H);
-        k_bn_copy_u32<<<8, 256, 0, c->stream>>>(reinterpret_cast<const uint32_t*>(m->act), fin + 2 * H, H / 4);
-        k_bn_copy_u32<<<1, 64, 0, c->stream>>>(reinterpret_cast<const uint32_t*>(sa), fin + 2 * H + H / 4, 1);
-        TI_LAUNCHED("k_bn_copy_u32 (trace)");
-    }
-    RC(ti_tern_gemv(c, m->lraw, m->lm.codes, m->lm.scales, m->act, m->xsum, C.vocab, H));
-    k_bn_logits<<<BN_AMAX_PARTS, 256, 0, c->stream>>>(m->lraw, sa, C.vocab, m->logits, m->amax_v, m->amax_i);
-    TI_LAUNCHED("k_bn_logits");
-    k_bn_argmax<<<1, BN_AMAX_PARTS, 0, c->stream>>>(m->amax_v, m->amax_i, BN_AMAX_PARTS, m->hist, m->dpos, C.max_ctx, m->rope,
-                                                    m->rope_cur, hd);
-    TI_LAUNCHED("k_bn_argmax");
-    return TI_OK;
+    return bonsai_logits(c, m, m->x, m->draw, sd);
 #undef RC
 }
 
@@ -1088,6 +1127,53 @@ extern "C" int ti_bonsai_decode(ti_ctx* c, ti_bonsai* m) {
     TI_CHECK_CTX(c);
     TI_REQUIRE(m, "ti_bonsai_decode: null model");
     return bonsai_step(c, m, true);
+}
+
+// T tokens hist[pos .. pos + T) at once: their KV rows, and (last) the logits and argmax of the
+// last one. The device position is left to the caller, except that the argmax advances it.
+static int bonsai_batch(ti_ctx* c, ti_bonsai* m, int pos, int T, bool last) {
+    const ti_bonsai_config& C = m->cfg;
+    const int H = C.hidden, I = C.intermediate, hd = C.head_dim, nHq = C.n_heads, nKv = C.n_kv_heads;
+    const int nq = nHq * hd, nkv = nKv * hd;
+    const ti_bb_rows R = {m->b.act, m->b.xsum, T};
+    const int8_t* act = reinterpret_cast<const int8_t*>(m->b.act);
+    float *sa = m->b.scales, *sb = sa + m->batch, *scl = sb + m->batch, *sd = scl + m->batch;
+    int rc;
+#define RC(x) do { rc = (x); if (rc) return rc; } while (0)
+    auto gemm = [&](int K, int n, TLin* const* w, float* const* out) {
+        const uint8_t* codes[3];
+        const float* scales[3];
+        long strides[3];
+        int Ns[3];
+        for (int i = 0; i < n; i++) {
+            codes[i] = w[i]->codes;
+            scales[i] = w[i]->scales;
+            strides[i] = Ns[i] = w[i]->N;
+        }
+        return ti_tern_gemm_mfma(c, act, m->b.xsum, K, T, n, codes, scales, out, strides, Ns);
+    };
+    for (int l = 0; l < C.layers; l++) {
+        BLayer& y = m->L[l];
+        RC(ti_bb_norm(c, R, m->b.x, m->b.d, sd, y.in_norm, C.rms_eps, H, m->hist + pos, l == 0 ? m->embed : nullptr, C.vocab, sa));
+        TLin* wq[3] = {&y.q, &y.k, &y.v};
+        float* oq[3] = {m->b.q, m->b.k, m->b.v};
+        RC(gemm(H, 3, wq, oq));
+        RC(ti_bb_rope(c, m->b.q, m->b.k, m->b.v, sa, y.q_norm, y.k_norm, m->rope + (size_t)pos * hd, C.rms_eps, m->b.qrot,
+                      y.kc + (size_t)pos * nkv, y.vc + (size_t)pos * nkv, T, nHq, nKv));
+        RC(ti_bb_attn(c, R, m->b.qrot, y.kc, y.vc, pos, nHq, nKv, m->b.po, m->b.pml, m->rowsplits, sb));
+        TLin* wo[1] = {&y.o};
+        RC(gemm(nq, 1, wo, &m->b.o));
+        RC(ti_bb_norm(c, R, m->b.x, m->b.o, sb, y.post_norm, C.rms_eps, H, nullptr, nullptr, 0, scl));
+        TLin* wg[2] = {&y.gate, &y.up};
+        float* og[2] = {m->b.g, m->b.u};
+        RC(gemm(H, 2, wg, og));
+        RC(ti_bb_swiglu(c, R, m->b.g, m->b.u, scl, I, sd));
+        TLin* wd[1] = {&y.down};
+        RC(gemm(I, 1, wd, &m->b.d));
+    }
+    if (!last) return TI_OK;
+    return bonsai_logits(c, m, m->b.x + (size_t)(T - 1) * H, m->b.d + (size_t)(T - 1) * H, sd + T - 1);
+#undef RC
 }
 
 // Prompt tokens ids[0..T) at positions pos.. (Model::forward per token, logits only for the
@@ -1100,8 +1186,16 @@ extern "C" int ti_bonsai_forward(ti_ctx* c, ti_bonsai* m, const int32_t* ids, in
                m->cfg.max_ctx);
     int rc;
     if (ids && (rc = ti_buf_write(c, m->hist, (size_t)pos * 4, ids, (size_t)T * 4))) return rc;
-    if ((rc = ti_bonsai_set_pos(c, m, pos))) return rc;
-    for (int t = 0; t < T; t++)
-        if ((rc = bonsai_step(c, m, t == T - 1))) return rc;
+    if (T == 1 || m->trace) {   // token by token: one token, or its fields are traced
+        if ((rc = ti_bonsai_set_pos(c, m, pos))) return rc;
+        for (int t = 0; t < T; t++)
+            if ((rc = bonsai_step(c, m, t == T - 1))) return rc;
+        return TI_OK;
+    }
+    if ((rc = ti_bonsai_set_pos(c, m, pos + T - 1))) return rc;   // the last token's, for its argmax
+    for (int t = 0; t < T; t += m->batch) {
+        const int n = T - t < m->batch ? T - t : m->batch;
+        if ((rc = bonsai_batch(c, m, pos + t, n, t + n == T))) return rc;
+    }
     return TI_OK;
 }
