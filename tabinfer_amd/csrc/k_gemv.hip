@@ -455,8 +455,6 @@ extern "C" int ti_group_dots_q4_q8(ti_ctx* c, const uint32_t* xq, const uint32_t
 // linearQ router: the activation scratch lives in the context (allocated once at
 // init), like the reference's _dp4/_dp4g buffers.
 int ti_quant_act_q8_async(ti_ctx* c, const float* x, uint32_t* xq, float* xs, int32_t* xsum, int groups);
-int ti_gemm_q4_q8_launch(ti_ctx* c, const uint32_t* xq, const float* xs, const uint32_t* pack, const uint16_t* scales,
-                         float* y, int T, int N, int K, int acc);
 int ti_fused_linear_launch(ti_ctx*, const float*, const uint32_t*, const uint16_t*, float*, int, int, int);
 int ti_fused_kmax(int lm);
 
@@ -469,11 +467,17 @@ extern "C" int ti_linear_q4(ti_ctx* c, const float* x, const uint32_t* pack, con
     TI_REQUIRE(al16(x) && al16(pack), "ti_linear_q4: x and pack must be 16-byte aligned");
     if (T == 1 && N >= 16384) return ti_gemv_q4_f32_launch(c, x, pack, scales, y, N, K, acc);
     if (T == 1 && K <= ti_fused_kmax(0)) return ti_fused_linear_launch(c, x, pack, scales, y, N, K, acc);
-    int rc = ti_quant_act_q8_async(c, x, c->act_q, c->act_s, nullptr, T * (K / 32));
-    if (rc) return rc;
+    int rc;
+    const bool shortb = ti_tgemm_ok(T, K) && reinterpret_cast<uintptr_t>(scales) % 16 == 0;
+    if (T > 1 && !shortb) {
+        // fragments in the same scratch: 2 bytes a code, but K <= TI_ACT_CAP / 4
+        TI_REQUIRE(ti_gemm_ok(K), "int4 GEMM: K=%d too large", K);
+        const TiFrag f = {c->act_q, c->act_s};
+        if ((rc = ti_quant_frag_launch(c, x, f, T, K))) return rc;
+        return ti_gemm_q4_launch(c, f, 1, &pack, &scales, &y, &N, T, K, acc);
+    }
+    if ((rc = ti_quant_act_q8_async(c, x, c->act_q, c->act_s, nullptr, T * (K / 32)))) return rc;
     if (T == 1) return ti_gemv_q4_q8_launch(c, c->act_q, c->act_s, pack, scales, y, N, K, acc);
-    if (ti_tgemm_ok(T, K) && reinterpret_cast<uintptr_t>(scales) % 16 == 0)
-        return ti_tgemm_launch(c, TgIn{c->act_q, c->act_s, nullptr, nullptr, 0.0f, nullptr}, 1, &pack, &scales, &y, &N, T, K,
-                               acc, nullptr);
-    return ti_gemm_q4_q8_launch(c, c->act_q, c->act_s, pack, scales, y, T, N, K, acc);
+    return ti_tgemm_launch(c, TgIn{c->act_q, c->act_s, nullptr, nullptr, 0.0f, nullptr}, 1, &pack, &scales, &y, &N, T, K,
+                           acc, nullptr);
 }

@@ -122,6 +122,21 @@ int ti_tern_gemm_mfma(ti_ctx* c, const int8_t* act, const int32_t* xsum, int K, 
                       const float* const* scales, float* const* outs, const long* strides, const int* Ns);
 int ti_tern_gemv_multi_norm(ti_ctx* c, const ti_tern_norm* nq, int K, int nmat, const uint8_t* const* codes,
                             const float* const* scales, float* const* outs, const int* Ns);
+// An activation [T][K] as the prompt GEMM reads it (k_gemm.hip): f16 codes [tile of 16 tokens]
+// [K / 32][64 lanes][8], and [tile][K / 32][32] floats: the tokens' scales, then -1032 * sum(codes)
+struct TiFrag {
+    uint32_t* xh;
+    float* sc;
+};
+bool ti_gemm_ok(int K);
+size_t ti_frag_words(int T, int K);
+size_t ti_frag_scales(int T, int K);
+int ti_quant_frag_launch(ti_ctx* c, const float* x, const TiFrag& f, int T, int K);
+int ti_norm_frag_launch(ti_ctx* c, const float* x, const uint16_t* w, float eps, const TiFrag& f, int T, int H);
+int ti_gemm_q4_launch(ti_ctx* c, const TiFrag& f, int nseg, const uint32_t* const* packs, const uint16_t* const* scs,
+                      float* const* ys, const int* Ns, int T, int K, int acc);
+int ti_gemm_gateup_launch(ti_ctx* c, const TiFrag& f, const uint32_t* gpack, const uint16_t* gsc, const uint32_t* upack,
+                          const uint16_t* usc, int I, int H, int T, const TiFrag& out);
 bool ti_tgemm_ok(int T, int K);
 bool ti_tgemm_norm_ok(int T, int K);
 bool ti_tnorm_ok(int K);

@@ -151,6 +151,7 @@ struct ti_qwen3 {
     uint32_t* xq;
     float* xs;
     int32_t* xsum;
+    TiFrag frag;          // the SwiGLU of a prompt as the down projection reads it
     float* psum;          // [16][256] RMSNorm partial sums of x (the T-token forward)
     uint32_t* hist;
     int* dpos;
@@ -298,6 +299,8 @@ extern "C" int ti_qwen3_create(ti_ctx* c, const ti_qwen3_config* cfg, ti_qwen3**
     const size_t kmax = (size_t)(H > I ? (H > nq ? H : nq) : (I > nq ? I : nq));   // widest GEMV input
     if (!rc) rc = mk(m, (void**)&m->xq, (size_t)T * kmax);                          // [T][kmax] int8 codes
     if (!rc) rc = mk(m, (void**)&m->xs, (size_t)T * kmax / 32 * 4);
+    if (!rc) rc = mk(m, (void**)&m->frag.xh, ti_frag_words(T, (int)kmax) * 4);
+    if (!rc) rc = mk(m, (void**)&m->frag.sc, ti_frag_scales(T, (int)kmax) * 4);
     if (!rc) rc = mk(m, (void**)&m->xsum, kmax / 16 * 4);
     if (!rc) rc = mk(m, (void**)&m->psum, 16 * 256 * 4);
     if (!rc) rc = mk(m, (void**)&m->hist, (size_t)(C.max_ctx + 1) * 4);
@@ -630,6 +633,12 @@ extern "C" int ti_qwen3_forward(ti_ctx* c, ti_qwen3* m, const int32_t* ids, int 
                        nq % 16 == 0 && nkv % 16 == 0 && I % 32 == 0;
     const bool fused_attn = ti_tattn_ok(T, nHq, nKv, hd);
     const bool norm_in = fused && T <= 4 && ti_tgemm_norm_ok(T, H);
+    // Longer prompts (and widths without a short-batch kernel): [rmsnorm + quantQ8T] [q/k/v]
+    // [attention] [quantQ8T] [o_proj + residual] [rmsnorm + quantQ8T] [gate/up + SiLU + quantQ8T]
+    // [down + residual] on the prompt GEMM (k_gemm.hip). A traced forward, whose fields hold the
+    // f32 SwiGLU, and a single token outside a decode step run operation by operation.
+    const bool prompt = !fused && T > 1 && !m->trace && ti_gemm_ok(H) && ti_gemm_ok(nq) && ti_gemm_ok(I);
+    const TiFrag cfrag = {c->act_q, c->act_s};
     if (norm_in) RC(ti_tsumsq_launch(c, m->x, m->psum, T, H));
     float* const pout = norm_in ? m->psum : nullptr;
     const TgIn codes_in = {c->act_q, c->act_s, nullptr, nullptr, 0.0f, nullptr};
@@ -649,6 +658,13 @@ extern "C" int ti_qwen3_forward(ti_ctx* c, ti_qwen3* m, const int32_t* ids, int 
                 RC(trace_put(c, m, l, TR_XN_S, c->act_s, T));
             }
             RC(ti_tgemm_launch(c, norm_in ? in_norm : codes_in, 3, packs, scs, ys, Ns, T, H, 0, nullptr));
+        } else if (prompt) {
+            const uint32_t* packs[3] = {y.q.pack, y.k.pack, y.v.pack};
+            const uint16_t* scs[3] = {y.q.sc, y.k.sc, y.v.sc};
+            float* ys[3] = {m->q, m->k, m->v};
+            const int Ns[3] = {nq, nkv, nkv};
+            RC(ti_norm_frag_launch(c, m->x, y.in_norm, C.rms_eps, cfrag, T, H));
+            RC(ti_gemm_q4_launch(c, cfrag, 3, packs, scs, ys, Ns, T, H, 0));
         } else {
             RC(ti_rmsnorm(c, m->x, y.in_norm, m->normed, T, H, C.rms_eps));
             RC(ti_linear_q4(c, m->normed, y.q.pack, y.q.sc, m->q, T, nq, H, 0));
@@ -684,6 +700,14 @@ extern "C" int ti_qwen3_forward(ti_ctx* c, ti_qwen3* m, const int32_t* ids, int 
             RC(trace_put(c, m, l, TR_S_Q, m->xq, T));
             RC(trace_put(c, m, l, TR_S_S, m->xs, T));
             RC(ti_tgemm_launch(c, attn_in, 1, &y.down.pack, &y.down.sc, &m->x, &H, T, I, 1, pout));
+            continue;
+        }
+        if (prompt) {
+            RC(ti_quant_frag_launch(c, m->attn, cfrag, T, nq));
+            RC(ti_gemm_q4_launch(c, cfrag, 1, &y.o.pack, &y.o.sc, &m->x, &H, T, nq, 1));
+            RC(ti_norm_frag_launch(c, m->x, y.post_norm, C.rms_eps, cfrag, T, H));
+            RC(ti_gemm_gateup_launch(c, cfrag, y.gate.pack, y.gate.sc, y.up.pack, y.up.sc, I, H, T, m->frag));
+            RC(ti_gemm_q4_launch(c, m->frag, 1, &y.down.pack, &y.down.sc, &m->x, &H, T, I, 1));
             continue;
         }
         RC(trace_put(c, m, l, TR_ATTN, m->attn, T));
