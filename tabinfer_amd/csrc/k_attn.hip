@@ -668,6 +668,8 @@ int ti_attn_decode_launch(ti_ctx* c, const float* qr, const uint32_t* kq, const 
     if ((long)T * nHq * nsplit > TI_ATTN_ROWSPLITS)
         return ti_fail(TI_ERR_INVALID, "ti_attn_decode_q8: T*nHq*nsplit = %ld > %d", (long)T * nHq * nsplit, TI_ATTN_ROWSPLITS);
     int G = nHq / nKv;
+    if (!dpos && ti_pattn_ok(T, nHq, nKv, hd))
+        return ti_pattn_launch(c, qr, kq, ks, vq, vs, out, nullptr, S, T, nHq, nKv, kvs);
     if (!dpos && T > 1 && hd == 128) {   // one pass over the keys for all T queries
         const int Smax = S + T - 1;
         const int want = (1024 + nKv - 1) / nKv;

@@ -1,0 +1,367 @@
+// k_pattn.hip — causal attention of a prompt's tokens over the int8 KV cache (attnBlock's T > 1 case,
+// models/qwen3.js:2534-2577), head_dim 128, both products on the matrix cores at f32 accuracy.
+//
+// Workgroup (4 waves): one KV head, one range of keys, 64 R query rows (row = token x query head of the
+// KV head); a wave owns 16 R rows and meets the others only over the staged keys. Key blocks of 64 are
+// staged in LDS as MFMA operands (f16 codes, exact), the next block's loads in flight meanwhile.
+//   - S^T = K Q^T, one v_mfma_f32_16x16x32_f16 per 32-dim scale group, 16 keys and q half: q = hi + lo in
+//     f16 (to 2^-22), each group's sum scaled by its key's scale in f32. Transposed, a lane's scores are
+//     those of one query row, keys 4j..4j+3 of each 16: the P operand of the second product as they
+//     stand, and the row's running maximum and sum live in its own four lanes.
+//   - O^T = V^T P^T with P times the V scale of (key, group), again split into f16 hi + lo. The scales
+//     are taken relative to the power of two under the range's largest of that group, and 2^10 up, so
+//     that hi lies in f16's normal range and what hi + lo lose is 2^-36 of the largest weight.
+// What bounds it is the VALU work of the weights (scale, mask, exponential, four scaled splits) and, with
+// 16 rows a wave, the LDS reads of the operands: with 32 rows each operand is read once for two products.
+// The ranges' partials (o, m, l; m in log2) are merged by k_pattn_merge, which also quantizes the output
+// into the o projection's fragments (k_gemm.hip) when asked.
+// 256 tokens x 16 heads over 4096 keys: 57.5 us with the merge, against 353 of k_attn_multi_q8 (P V as f32
+// FMAs, a workgroup per 16 rows); error against 64 bits 2.4e-7, against 2.5e-7.
+#include "ti_dev.h"
+
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+constexpr int HD = 128, NG = HD / 32, KB = 64;         // KB: keys of a staged block
+constexpr int VSTRIDE = 65;                            // 16-byte pieces of a V operand tile (1 of padding: writes of
+                                                       // eight tiles would meet in one bank)
+constexpr uint32_t WUP = 10;                           // log2 of the weights' factor
+constexpr float MLOW = -3.0e38f;
+
+struct PattnArgs {
+    const float* qr;
+    const uint8_t* kq;
+    const float* ks;
+    const uint8_t* vq;
+    const float* vs;
+    float* po;
+    float* pml;
+    int S0, T, nHq, nKv, G, nsplit, per, nblk;         // S0: keys token 0 sees; per: keys of a range (multiple of KB)
+    int kvs;                                           // code slots of a cached position
+};
+
+struct PattnLds {
+    ti_h8 k[KB / 16][NG][64];                          // [16 keys][group][lane]: key lane % 16, dims 8 (lane / 16)..
+    ti_h8 v[KB / 32][8][VSTRIDE];                      // [32 keys][16 dims][lane]: dim lane % 16, keys 4j.., 16 + 4j..
+    float ks[NG][KB], vs[NG][KB];
+    float vmax[4][NG];
+};
+
+// 4 x 4 bytes: in, w[r] = row r's four bytes; out, w[e] = byte e of rows 0..3
+__device__ __forceinline__ void tr4_bytes(uint32_t (&w)[4]) {
+    const uint32_t a = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u);   // r0b0 r1b0 r0b1 r1b1
+    const uint32_t b = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);   // r0b2 r1b2 r0b3 r1b3
+    const uint32_t c = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u);
+    const uint32_t d = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
+    w[0] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+    w[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+    w[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
+    w[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
+}
+
+template <int R>
+__global__ __launch_bounds__(256, 2) void k_pattn(PattnArgs a) {
+    __shared__ PattnLds L;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = lane & 15, j = lane >> 4;
+    // KV head fastest: an XCD (every eighth workgroup) keeps to few heads' keys
+    const int hk = blockIdx.x % a.nKv, blk = (blockIdx.x / a.nKv) % a.nblk, split = blockIdx.x / (a.nKv * a.nblk);
+    const int nrows = a.G * a.T;
+    const int row0 = blk * 64 * R + wave * 16 * R;
+    const int wgtop = min((blk + 1) * 64 * R, nrows) - 1;
+    const int c0 = split * a.per;
+    const int c1 = min(a.S0 + wgtop / a.G, c0 + a.per);    // keys [c0, c1) that any row of the workgroup sees
+    const size_t code_row = (size_t)a.kvs * HD, scale_row = (size_t)a.nKv * NG;
+    const uint8_t* kp = a.kq + hk * HD;
+    const uint8_t* vp = a.vq + hk * HD;
+    const float* ksp = a.ks + hk * NG;
+    const float* vsp = a.vs + hk * NG;
+    const float sscale = 1.44269504088896341f / (127.0f * sqrtf((float)HD));
+
+    // a block's loads of this thread: K 2 x 16 codes of key 16 wave + m; V 2 blocks of 4 keys x 4 dims; one scale each
+    uint4 kr[2];
+    uint32_t vr[2][4];
+    float ksr, vsr;
+    const int vdb = lane & 31, vkb = (lane >> 5) + 2 * wave;
+    auto load = [&](int t0) {
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            kr[u] = *reinterpret_cast<const uint4*>(kp + min(t0 + 16 * wave + m, c1 - 1) * code_row + 16 * (j + 4 * u));
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                vr[u][r] = *reinterpret_cast<const uint32_t*>(vp + min(t0 + 4 * (vkb + 8 * u) + r, c1 - 1) * code_row + 4 * vdb);
+        const size_t s = min(t0 + (tid >> 2), c1 - 1) * scale_row + (tid & 3);
+        ksr = ksp[s];
+        vsr = vsp[s];
+    };
+    if (c0 < c1) load(c0);
+
+    // the range's largest V scale of each group -> the power of two under it
+    float gmax = 0.0f;
+    for (int t = c0 + (tid >> 2); t < c1; t += 64) gmax = fmaxf(gmax, vsp[t * scale_row + (tid & 3)]);
+#pragma unroll
+    for (int o = 4; o < 64; o <<= 1) gmax = fmaxf(gmax, ti_xor(gmax, o));
+    if (lane < NG) L.vmax[wave][lane] = gmax;
+    __syncthreads();
+    auto pow2 = [&](int g) {
+        const float v = fmaxf(fmaxf(L.vmax[0][g], L.vmax[1][g]), fmaxf(L.vmax[2][g], L.vmax[3][g]));
+        const uint32_t e = __builtin_bit_cast(uint32_t, v) & 0x7f800000u;
+        return min(max(e, 0x08000000u), 0x7e000000u);
+    };
+    // 2^(WUP - e) for the group this thread stages
+    const float vdown = __builtin_bit_cast(float, 0x7f000000u - pow2(tid & 3) + (WUP << 23));
+
+    float neg = -1.0f;                                     // opaque: w - hi as one v_fma_mix, not convert and subtract
+    asm("" : "+s"(neg));
+    // Q operands: this wave's row m of each 16, dims 32 g + 8 j.., hi and lo; and the keys the row sees
+    ti_h8 qh[R][NG], ql[R][NG];
+    int lim[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int gr = row0 + 16 * r + m;
+        const bool ok = gr < nrows;
+        const int t = ok ? gr / a.G : 0, h = ok ? gr % a.G : 0;
+        lim[r] = ok ? min(c1, a.S0 + t) : 0;
+        const float* q = a.qr + ((size_t)t * a.nHq + hk * a.G + h) * HD;
+#pragma unroll
+        for (int g = 0; g < NG; g++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float v = ok ? q[32 * g + 8 * j + e] : 0.0f;
+                const _Float16 hi = (_Float16)v;
+                qh[r][g][e] = hi;
+                ql[r][g][e] = (_Float16)fmaf((float)hi, neg, v);
+            }
+    }
+    // every row of the wave sees the keys below this
+    const int all = row0 + 16 * R <= nrows ? min(c1, a.S0 + row0 / a.G) : 0;
+
+    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    v4f o[R][8];
+    float mx[R], l[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        mx[r] = MLOW;
+        l[r] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < 8; d++) o[r][d] = zero;
+    }
+    for (int t0 = c0; t0 < c1; t0 += KB) {
+        __syncthreads();                                   // the last block is read
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int c = j + 4 * u;
+            L.k[wave][c >> 1][(c & 1) * 32 + m] = ti_i8x8_h8(kr[u].x, kr[u].y);
+            L.k[wave][c >> 1][(c & 1) * 32 + 16 + m] = ti_i8x8_h8(kr[u].z, kr[u].w);
+            const int kb = vkb + 8 * u, kk = kb & 7;       // 4-key block of its 32 keys
+            tr4_bytes(vr[u]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                ti_h2 h0, h1;
+                ti_i8x4_h2x2(vr[u][e], h0, h1);
+                ti_h8* p = &L.v[kb >> 3][vdb >> 2][(kk & 3) * 16 + 4 * (vdb & 3) + e];
+                reinterpret_cast<uint2*>(p)[kk >> 2] = make_uint2(__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1));
+            }
+        }
+        L.ks[tid & 3][tid >> 2] = ksr;
+        L.vs[tid & 3][tid >> 2] = vsr * vdown;
+        __syncthreads();
+        if (t0 + KB < c1) load(t0 + KB);
+        TI_ISSUE_FENCE();
+#pragma unroll 1
+        for (int h = 0; h < KB / 32; h++) {                // 32 keys
+            const int k0 = t0 + 32 * h;
+            if (k0 >= c1) break;                           // workgroup-uniform
+            v4f s[R][2];
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+#pragma unroll
+                for (int r = 0; r < R; r++) s[r][b] = zero;
+#pragma unroll
+                for (int g = 0; g < NG; g++) {
+                    const ti_h8 kk = L.k[2 * h + b][g][lane];
+                    const v4f sc = *reinterpret_cast<const v4f*>(&L.ks[g][32 * h + 16 * b + 4 * j]);
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        v4f d = __builtin_amdgcn_mfma_f32_16x16x32_f16(kk, qh[r][g], zero, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(kk, ql[r][g], d, 0, 0, 0);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) s[r][b][i] = fmaf(d[i], sc[i], s[r][b][i]);
+                    }
+                }
+            }
+            const bool masked = k0 + 32 > all;             // wave-uniform
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                float tm = MLOW;
+#pragma unroll
+                for (int b = 0; b < 2; b++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        s[r][b][i] = s[r][b][i] * sscale;
+                        if (masked) s[r][b][i] = k0 + 16 * b + 4 * j + i < lim[r] ? s[r][b][i] : MLOW;
+                        tm = fmaxf(tm, s[r][b][i]);
+                    }
+                tm = fmaxf(tm, ti_xor(tm, 16));
+                tm = fmaxf(tm, ti_xor(tm, 32));
+                const float mn = fmaxf(mx[r], tm);
+                if (__any(mn > mx[r])) {                   // rare once the first blocks are in
+                    const float alpha = __builtin_amdgcn_exp2f(mx[r] - mn);
+                    l[r] = l[r] * alpha;
+#pragma unroll
+                    for (int d = 0; d < 8; d++) o[r][d] = o[r][d] * alpha;
+                    mx[r] = mn;
+                }
+#pragma unroll
+                for (int b = 0; b < 2; b++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        float p = __builtin_amdgcn_exp2f(s[r][b][i] - mx[r]);
+                        if (masked) p = k0 + 16 * b + 4 * j + i < lim[r] ? p : 0.0f;
+                        l[r] += p;
+                        s[r][b][i] = p;
+                    }
+            }
+#pragma unroll
+            for (int g = 0; g < NG; g++) {
+                const v4f v0 = *reinterpret_cast<const v4f*>(&L.vs[g][32 * h + 4 * j]);
+                const v4f v1 = *reinterpret_cast<const v4f*>(&L.vs[g][32 * h + 16 + 4 * j]);
+                ti_h8 ph[R], pl[R];
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        const float w0 = e < 4 ? s[r][0][e] * v0[e] : s[r][1][e - 4] * v1[e - 4];
+                        const float w1 = e < 4 ? s[r][0][e + 1] * v0[e + 1] : s[r][1][e - 3] * v1[e - 3];
+                        // opaque: else lo may be taken from a hi that was rounded from the unrounded product
+                        uint32_t hp = __builtin_bit_cast(uint32_t, ti_h2{(_Float16)w0, (_Float16)w1});
+                        asm("" : "+v"(hp));
+                        const ti_h2 hi = __builtin_bit_cast(ti_h2, hp);
+                        ph[r][e] = hi[0];
+                        ph[r][e + 1] = hi[1];
+                        pl[r][e] = (_Float16)fmaf((float)hi[0], neg, w0);
+                        pl[r][e + 1] = (_Float16)fmaf((float)hi[1], neg, w1);
+                    }
+#pragma unroll
+                for (int d = 2 * g; d < 2 * g + 2; d++) {
+                    const ti_h8 vv = L.v[h][d][lane];
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        o[r][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, ph[r], o[r][d], 0, 0, 0);
+                        o[r][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, pl[r], o[r][d], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int gr = row0 + 16 * r + m;
+        float lt = l[r];
+        lt += ti_xor(lt, 16);
+        lt += ti_xor(lt, 32);
+        if (gr >= nrows) continue;
+        const int t = gr / a.G, hq = hk * a.G + gr % a.G;
+        const size_t slot = ((size_t)t * a.nHq + hq) * a.nsplit + split;
+#pragma unroll
+        for (int d = 0; d < 8; d++)
+            *reinterpret_cast<v4f*>(a.po + slot * HD + 16 * d + 4 * j) = o[r][d] * __builtin_bit_cast(float, pow2(d / 2) - (WUP << 23));
+        if (j == 0) {
+            a.pml[2 * slot] = mx[r];
+            a.pml[2 * slot + 1] = lt;
+        }
+    }
+}
+
+// The ranges' partials of a (token, head) -> its output row, a wave each. FRAG: quantized into the o
+// projection's fragments (tokens past T of the last tile of 16 as zeros); else out [T][nHq][128]. Lane
+// l holds dims 8 (l / 4) + l % 4 and + 4, neighbours in the fragment.
+template <bool FRAG>
+__global__ __launch_bounds__(256) void k_pattn_merge(const float* __restrict__ po, const float* __restrict__ pml,
+                                                     float* __restrict__ out, uint32_t* __restrict__ xh,
+                                                     float* __restrict__ xsc, int T, int nHq, int nsplit, int rows) {
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;                               // wave-uniform
+    const int t = row / nHq, h = row % nHq;
+    const int sl = lane >> 2, d = 8 * sl + (lane & 3);
+    float v0 = 0.0f, v1 = 0.0f;
+    if (t < T) {
+        const float* p = po + (size_t)row * nsplit * HD + d;
+        const float* ml = pml + (size_t)row * nsplit * 2;
+        const float mi = lane < nsplit ? ml[2 * lane] : MLOW, li = lane < nsplit ? ml[2 * lane + 1] : 0.0f;   // nsplit <= 64
+        const float w = __builtin_amdgcn_exp2f(mi - ti_wave_max(mi));
+        const float lt = ti_wave_sum(li * w);
+        for (int i0 = 0; i0 < nsplit; i0 += 8) {
+            float a[8], b[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const int i = min(i0 + k, nsplit - 1);
+                a[k] = p[(size_t)i * HD];
+                b[k] = p[(size_t)i * HD + 4];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const float f = i0 + k < nsplit ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), i0 + k)) : 0.0f;
+                v0 = fmaf(a[k], f, v0);
+                v1 = fmaf(b[k], f, v1);
+            }
+        }
+        const float inv = 127.0f * lt;
+        v0 = v0 / inv;
+        v1 = v1 / inv;
+    }
+    if constexpr (!FRAG) {
+        out[(size_t)row * HD + d] = v0;
+        out[(size_t)row * HD + d + 4] = v1;
+    } else {
+        float mx = fmaxf(fabsf(v0), fabsf(v1));
+        mx = fmaxf(mx, ti_xor(mx, 1));
+        mx = fmaxf(mx, ti_xor(mx, 2));
+        mx = fmaxf(mx, ti_xor(mx, 4));
+        mx = fmaxf(mx, ti_xor(mx, 8));
+        const float scale = mx / 127.0f;
+        const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
+        const ti_h2 q = {(_Float16)q8_code(v0, inv), (_Float16)q8_code(v1, inv)};
+        const size_t f = (size_t)(t >> 4) * nHq * NG + h * NG + (sl >> 2);
+        xh[(f * 64 + 16 * (sl & 3) + (t & 15)) * 4 + (lane & 3)] = __builtin_bit_cast(uint32_t, q);
+        if ((lane & 15) == 0) xsc[f * 16 + (t & 15)] = scale;
+    }
+}
+
+}  // namespace
+
+// 32 rows or fewer would leave half of a workgroup's waves idle: the short kernels keep them
+bool ti_pattn_ok(int T, int nHq, int nKv, int hd) { return hd == HD && T > 1 && nHq / nKv * T > 32; }
+
+// queries T at contexts S0, S0 + 1, ...: out [T][nHq][128], or (frag) the o projection's fragments
+int ti_pattn_launch(ti_ctx* c, const float* qr, const uint32_t* kq, const float* ks, const uint32_t* vq, const float* vs,
+                    float* out, const TiFrag* frag, int S0, int T, int nHq, int nKv, int kvs) {
+    const int G = nHq / nKv, nrows = G * T, Smax = S0 + T - 1;
+    const int R = nrows > 64 ? 2 : 1;
+    const int nblk = (nrows + 64 * R - 1) / (64 * R);
+    // key ranges: two workgroups a CU, of at least two blocks, and the merge reads every range's rows
+    long ns = (2L * c->cus + (long)nKv * nblk - 1) / ((long)nKv * nblk);
+    const long kb = (Smax + KB - 1) / KB;
+    if (ns > (kb + 1) / 2) ns = (kb + 1) / 2;
+    if (ns > 64) ns = 64;
+    if (ns * T * nHq > TI_ATTN_ROWSPLITS) ns = TI_ATTN_ROWSPLITS / ((long)T * nHq);
+    if (ns < 1) ns = 1;
+    const int per = (int)((kb + ns - 1) / ns) * KB;
+    const int nsplit = (Smax + per - 1) / per;
+    PattnArgs a = {qr, reinterpret_cast<const uint8_t*>(kq), ks, reinterpret_cast<const uint8_t*>(vq), vs, c->attn_po, c->attn_ml,
+                   S0, T, nHq, nKv, G, nsplit, per, nblk, kvs};
+    const unsigned grid = (unsigned)((long)nKv * nblk * nsplit);
+    if (R == 2) k_pattn<2><<<grid, 256, 0, c->stream>>>(a);
+    else k_pattn<1><<<grid, 256, 0, c->stream>>>(a);
+    TI_LAUNCHED("k_pattn");
+    const int rows = (frag ? (T + 15) / 16 * 16 : T) * nHq;
+    if (frag) k_pattn_merge<true><<<(rows + 3) / 4, 256, 0, c->stream>>>(c->attn_po, c->attn_ml, nullptr, frag->xh, frag->sc, T, nHq, nsplit, rows);
+    else k_pattn_merge<false><<<(rows + 3) / 4, 256, 0, c->stream>>>(c->attn_po, c->attn_ml, out, nullptr, nullptr, T, nHq, nsplit, rows);
+    TI_LAUNCHED("k_pattn_merge");
+    return TI_OK;
+}

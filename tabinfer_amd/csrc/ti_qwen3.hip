@@ -634,11 +634,12 @@ extern "C" int ti_qwen3_forward(ti_ctx* c, ti_qwen3* m, const int32_t* ids, int 
     const bool fused_attn = ti_tattn_ok(T, nHq, nKv, hd);
     const bool norm_in = fused && T <= 4 && ti_tgemm_norm_ok(T, H);
     // Longer prompts (and widths without a short-batch kernel): [rmsnorm + quantQ8T] [q/k/v]
-    // [attention] [quantQ8T] [o_proj + residual] [rmsnorm + quantQ8T] [gate/up + SiLU + quantQ8T]
-    // [down + residual] on the prompt GEMM (k_gemm.hip). A traced forward, whose fields hold the
+    // [attention] [merge + quantQ8T] [o_proj + residual] [rmsnorm + quantQ8T]
+    // [gate/up + SiLU + quantQ8T] [down + residual] (k_gemm.hip, k_pattn.hip). A traced forward, whose fields hold the
     // f32 SwiGLU, and a single token outside a decode step run operation by operation.
     const bool prompt = !fused && T > 1 && !m->trace && ti_gemm_ok(H) && ti_gemm_ok(nq) && ti_gemm_ok(I);
     const TiFrag cfrag = {c->act_q, c->act_s};
+    const bool pattn = prompt && ti_pattn_ok(T, nHq, nKv, hd);   // writes the o projection's fragments itself
     if (norm_in) RC(ti_tsumsq_launch(c, m->x, m->psum, T, H));
     float* const pout = norm_in ? m->psum : nullptr;
     const TgIn codes_in = {c->act_q, c->act_s, nullptr, nullptr, 0.0f, nullptr};
@@ -678,8 +679,11 @@ extern "C" int ti_qwen3_forward(ti_ctx* c, ti_qwen3* m, const int32_t* ids, int 
             RC(ti_rope_qk(c, m->q, y.q_norm, m->qr, T, nHq, hd, pos, C.rope_theta, C.rms_eps));
             RC(ti_rope_qk(c, m->k, y.k_norm, m->kr, T, nKv, hd, pos, C.rope_theta, C.rms_eps));
             RC(ti_kv_write_launch(c, m->kr, m->v, y.kq, y.ks, y.vq, y.vs, T, nKv, hd, pos, m->kvs));
-            RC(ti_attn_decode_launch(c, m->qr, y.kq, y.ks, y.vq, y.vs, m->attn, pos + 1, T, nHq, nKv, hd, 0, nullptr, 0,
-                                     m->kvs));
+            if (pattn)
+                RC(ti_pattn_launch(c, m->qr, y.kq, y.ks, y.vq, y.vs, nullptr, &cfrag, pos + 1, T, nHq, nKv, m->kvs));
+            else
+                RC(ti_attn_decode_launch(c, m->qr, y.kq, y.ks, y.vq, y.vs, m->attn, pos + 1, T, nHq, nKv, hd, 0, nullptr, 0,
+                                         m->kvs));
         }
         RC(trace_put(c, m, l, TR_Q, m->q, T));
         RC(trace_put(c, m, l, TR_K, m->k, T));
@@ -703,7 +707,7 @@ extern "C" int ti_qwen3_forward(ti_ctx* c, ti_qwen3* m, const int32_t* ids, int 
             continue;
         }
         if (prompt) {
-            RC(ti_quant_frag_launch(c, m->attn, cfrag, T, nq));
+            if (!pattn) RC(ti_quant_frag_launch(c, m->attn, cfrag, T, nq));
             RC(ti_gemm_q4_launch(c, cfrag, 1, &y.o.pack, &y.o.sc, &m->x, &H, T, nq, 1));
             RC(ti_norm_frag_launch(c, m->x, y.post_norm, C.rms_eps, cfrag, T, H));
             RC(ti_gemm_gateup_launch(c, cfrag, y.gate.pack, y.gate.sc, y.up.pack, y.up.sc, I, H, T, m->frag));
