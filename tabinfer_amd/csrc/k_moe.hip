@@ -12,6 +12,7 @@
 // activation words packed in the same order; the +4 offset is removed once per group from
 // the activation sum. The int32 group dot is the same integer in any element order.
 #include "ti_dev.h"
+#include "ti_moe.h"
 
 namespace {
 
@@ -135,8 +136,9 @@ __global__ __launch_bounds__(64) void k_router(const float* __restrict__ logits,
 }
 
 // the router (workgroups 0 .. T-1, one per token) and, in the same launch, quantAct8 of
-// the normed rows (the remaining workgroups, a 32-group per thread, words in
-// k_moe_gemm_q3's element order): the two do not depend on each other
+// the normed rows (the remaining workgroups, a 32-group per thread): the two do not depend on each
+// other. Codes as words in k_moe_gemm_q3's element order, or (F16) as the rows of k_moe_gemm.
+template <bool F16>
 __global__ __launch_bounds__(64) void k_router_quant(const float* __restrict__ logits, const float* __restrict__ bias,
                                                      int nE, int topk, int32_t* __restrict__ idx, float* __restrict__ wt,
                                                      int T, const float* __restrict__ x, uint32_t* __restrict__ xq,
@@ -149,31 +151,24 @@ __global__ __launch_bounds__(64) void k_router_quant(const float* __restrict__ l
     if (gi >= ng) return;
     float v[32];
     load32(x + (size_t)gi * 32, v);
-    q8_group<true>(v, xq + (size_t)gi * 8, xs + gi, nullptr);
+    if constexpr (!F16) {
+        q8_group<true>(v, xq + (size_t)gi * 8, xs + gi, nullptr);
+    } else {
+        float mx = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 32; i++) mx = fmaxf(mx, fabsf(v[i]));
+        const float scale = mx / 127.0f;
+        const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
+        xs[gi] = scale;
+        ti_h8 h[4];
+#pragma unroll
+        for (int i = 0; i < 32; i++) h[moe_slot(i) / 8][moe_slot(i) % 8] = (_Float16)q8_code(v[i], inv);
+#pragma unroll
+        for (int k = 0; k < 4; k++) reinterpret_cast<ti_h8*>(xq)[(size_t)gi * 4 + k] = h[k];
+    }
 }
 
 // ---- decode: pair-indexed GEMV with the f32 activation ----------------------------
-// A group's (q3 + 4) codes as bytes, q[c] byte i = element 8i + c. Elements 4t + r
-// (r = 0..3, t = 0..7) take plane bit positions 4t + r; gathering plane b's bits of one r
-// beside each other gives X_r with element 4t + r's code in nibble t (bits 4t + r + b for
-// r < 2, shifted down by 2 for r >= 2 so nothing leaves the word), then q[4h + r] is
-// nibbles h, h+2, h+4, h+6 of X_r, one per byte. 36 VALU operations per 32 codes.
-__device__ __forceinline__ void q3_cols(uint32_t b0, uint32_t b1, uint32_t b2, uint32_t (&q)[8]) {
-    constexpr uint32_t M = 0x11111111u, B = 0x07070707u;
-    const uint32_t x0 = (b0 & M) | ((b1 & M) << 1) | ((b2 & M) << 2);
-    const uint32_t x1 = (b0 & (M << 1)) | ((b1 & (M << 1)) << 1) | ((b2 & (M << 1)) << 2);
-    const uint32_t x2 = ((b0 & (M << 2)) >> 2) | ((b1 & (M << 2)) >> 1) | (b2 & (M << 2));
-    const uint32_t x3 = ((b0 & (M << 3)) >> 2) | ((b1 & (M << 3)) >> 1) | (b2 & (M << 3));
-    q[0] = x0 & B;
-    q[4] = (x0 >> 4) & B;
-    q[1] = (x1 >> 1) & B;
-    q[5] = (x1 >> 5) & B;
-    q[2] = x2 & B;
-    q[6] = (x2 >> 4) & B;
-    q[3] = (x3 >> 1) & B;
-    q[7] = (x3 >> 5) & B;
-}
-
 // f32 activation group as exact fixed point (as k_gemv_q4_f32): x_j = X_j * 2^(ex-22),
 // X = l2*65536 + l1*256 + l0 with signed int8 limbs, words in q3_cols's element order
 struct Limbs {
@@ -802,6 +797,12 @@ __global__ void k_moe_combine(float* __restrict__ x, const float* __restrict__ o
 
 static inline bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
+// From five pairs an expert on the matrix cores win; below, their 16-pair tile is mostly padding and the
+// row kernels, which take a pair at a time, do less (block of 2048 x 1792, top-4 of 32 experts, us row kernels /
+// matrix cores: 2 pairs an expert 58 / 72, 4 75.7 / 78.2, 5 85.4 / 82.4, 16 186 / 120, 20 227 / 140; 512 x 512, 16 experts,
+// 25 pairs 73.9 / 32.6).
+static bool ti_moe_mfma(long P, int nE) { return P >= 5L * nE; }
+
 extern "C" int ti_requant43(ti_ctx* c, const uint32_t* pack4, const uint16_t* sc4, int rows, int K, uint32_t* p3,
                             uint16_t* s3) {
     TI_CHECK_CTX(c);
@@ -854,7 +855,13 @@ extern "C" int ti_moe_gemm_q3(ti_ctx* c, const float* src, int src_rows, const u
     // quantAct8 (lfm25.js:1487-1494): per row, per 32-group int8 into the context's scratch,
     // words in the GEMM's element order (k_router_quant with no router workgroups)
     const int nq = src_rows * (K / 32);
-    k_router_quant<<<(unsigned)((nq + 63) / 64), 64, 0, c->stream>>>(nullptr, nullptr, 0, 0, nullptr, nullptr, 0, src,
+    if (ti_moe_mfma(P, nE)) {
+        k_router_quant<true><<<(unsigned)((nq + 63) / 64), 64, 0, c->stream>>>(nullptr, nullptr, 0, 0, nullptr, nullptr, 0, src,
+                                                                               c->act_q, c->act_s, nq);
+        TI_LAUNCHED("k_router_quant (quantizer only)");
+        return ti_moe_gemm_launch(c, reinterpret_cast<uint16_t*>(c->act_q), c->act_s, p3, s3, ridx, y, P, N, K, src_div, nE);
+    }
+    k_router_quant<false><<<(unsigned)((nq + 63) / 64), 64, 0, c->stream>>>(nullptr, nullptr, 0, 0, nullptr, nullptr, 0, src,
                                                                      c->act_q, c->act_s, nq);
     TI_LAUNCHED("k_router_quant (quantizer only)");
     dim3 grid((unsigned)((N + 15) / 16), (unsigned)nE);
@@ -905,7 +912,22 @@ extern "C" int ti_moe_prefill_q3(ti_ctx* c, float* x, const float* normed, const
     TI_REQUIRE(al16(normed) && al16(gate) && al16(up) && al16(act),
                "ti_moe_prefill_q3: normed, gate, up and act must be 16-byte aligned");
     const int nq = T * (H / 32);
-    k_router_quant<<<(unsigned)(T + (nq + 63) / 64), 64, 0, c->stream>>>(logits, bias, nE, topk, idx, wt, T, normed,
+    const long th = (long)T * H;
+    if (ti_moe_mfma(P, nE)) {
+        uint16_t* xh = reinterpret_cast<uint16_t*>(c->act_q);
+        k_router_quant<true><<<(unsigned)(T + (nq + 63) / 64), 64, 0, c->stream>>>(logits, bias, nE, topk, idx, wt, T, normed,
+                                                                                   c->act_q, c->act_s, nq);
+        TI_LAUNCHED("k_router_quant");
+        int rc;
+        if ((rc = ti_moe_gateup_launch(c, xh, c->act_s, w1p, w1s, w3p, w3s, idx, gate, up, act, c->moe_q, c->moe_s, (int)P, I, H,
+                                       topk, nE)))
+            return rc;
+        if ((rc = ti_moe_gemm_launch(c, c->moe_q, c->moe_s, w2p, w2s, idx, out, (int)P, H, I, 1, nE))) return rc;
+        k_moe_combine<<<(unsigned)((th + 255) / 256), 256, 0, c->stream>>>(x, out, wt, H, topk, th);
+        TI_LAUNCHED("k_moe_combine");
+        return TI_OK;
+    }
+    k_router_quant<false><<<(unsigned)(T + (nq + 63) / 64), 64, 0, c->stream>>>(logits, bias, nE, topk, idx, wt, T, normed,
                                                                           c->act_q, c->act_s, nq);
     TI_LAUNCHED("k_router_quant");
     const int spec = 2 * P >= nE;
@@ -920,7 +942,6 @@ extern "C" int ti_moe_prefill_q3(ti_ctx* c, float* x, const float* normed, const
     if (I <= 2048) k_moe_gemm_q3<1><<<g2, 256, 0, c->stream>>>(c->act_q, c->act_s, w2p, w2s, idx, out, (int)P, H, I, 1, spec, w2p, w2s, out);
     else k_moe_gemm_q3<2><<<g2, 256, 0, c->stream>>>(c->act_q, c->act_s, w2p, w2s, idx, out, (int)P, H, I, 1, spec, w2p, w2s, out);
     TI_LAUNCHED("k_moe_gemm_q3 (w2)");
-    const long th = (long)T * H;
     k_moe_combine<<<(unsigned)((th + 255) / 256), 256, 0, c->stream>>>(x, out, wt, H, topk, th);
     TI_LAUNCHED("k_moe_combine");
     return TI_OK;

@@ -22,13 +22,15 @@ struct ti_ctx {
     // persistent scratch (allocated at init, never reallocated, so calls may be
     // captured into graphs): int8 activation for the linearQ router, split-KV
     // partials, argmax partials.
-    uint32_t* act_q;      // [TI_ACT_CAP/4 * TI_ACT_TMAX]
+    uint32_t* act_q;      // [TI_ACT_CAP/2 * TI_ACT_TMAX]: codes as bytes, or as f16
     float* act_s;         // [TI_ACT_CAP/32 * TI_ACT_TMAX]
     int32_t* act_sum;     // [TI_ACT_CAP/16]
     float* attn_po;       // split-KV partial outputs
     float* attn_ml;       // split-KV (m, l)
     float* amax_v;        // argmax partial values
     uint32_t* amax_i;     // argmax partial indices
+    uint16_t* moe_q;      // the experts' quantized SwiGLU, as f16, while act_q is still read
+    float* moe_s;
     uint32_t* moe_cnt;    // MoE counting sort: counts / offsets / fill / sorted index
     uint32_t* moe_off;
     uint32_t* moe_fill;

@@ -30,7 +30,7 @@ extern "C" int ti_device_count(int* n) {
 // the stream, the host struct. Used by ti_shutdown and by every ti_init error path.
 static void destroy_ctx(ti_ctx* c) {
     void* ps[] = {c->act_q, c->act_s, c->act_sum, c->attn_po, c->attn_ml, c->amax_v, c->amax_i,
-                  c->moe_cnt, c->moe_off, c->moe_fill, c->moe_sidx, c->tg_part, c->qkv_pub, c->sync};
+                  c->moe_q, c->moe_s, c->moe_cnt, c->moe_off, c->moe_fill, c->moe_sidx, c->tg_part, c->qkv_pub, c->sync};
     for (void* p : ps) if (p) (void)hipFree(p);
     for (int i = 0; i < 64; i++) if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -67,7 +67,9 @@ extern "C" int ti_init(int device, ti_ctx** out) {
         if (e != hipSuccess) { c->ev[i] = nullptr; destroy_ctx(c); return ti_hip_fail(e, "hipEventCreate"); }
     }
     struct { void** p; size_t bytes; } allocs[] = {
-        {(void**)&c->act_q, (size_t)TI_ACT_CAP * TI_ACT_TMAX},
+        {(void**)&c->act_q, (size_t)TI_ACT_CAP * TI_ACT_TMAX * 2},
+        {(void**)&c->moe_q, (size_t)TI_ACT_CAP * TI_ACT_TMAX * 2},
+        {(void**)&c->moe_s, (size_t)TI_ACT_CAP / 32 * TI_ACT_TMAX * 4},
         {(void**)&c->act_s, (size_t)TI_ACT_CAP / 32 * TI_ACT_TMAX * 4},
         {(void**)&c->act_sum, (size_t)TI_ACT_CAP / 16 * 4},
         {(void**)&c->attn_po, (size_t)TI_ATTN_ROWSPLITS * TI_ATTN_HD_MAX * 4},
