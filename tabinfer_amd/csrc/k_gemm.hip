@@ -305,22 +305,50 @@ __global__ __launch_bounds__(256) void k_quant_frag(const float* __restrict__ x,
 }
 
 // RMSNorm (the reference's 256 strided partials and tree, as k_rmsnorm) + quantQ8 -> fragments;
-// a workgroup per token
+// a workgroup per token. KU: H = 256 KU, every load issued before the first sum waits (2048 wide, 256
+// tokens: 6.0 -> 4.9 us); KU = 0: any H.
+template <int KU>
 __global__ __launch_bounds__(256) void k_norm_frag(const float* __restrict__ x, const uint16_t* __restrict__ nw, float eps,
-                                                   ti_h8* __restrict__ xh, float* __restrict__ xsc, int T, int H) {
+                                                   ti_h8* __restrict__ xh, float* __restrict__ xsc, int T, int Hany) {
     __shared__ float red[256];
+    constexpr int NC = KU ? (KU + 7) / 8 : 1;              // 8-element chunks of a thread
+    const int H = KU ? 256 * KU : Hany;
     const int tok = blockIdx.x, G = H / 32, t = threadIdx.x;
     const size_t f0 = (size_t)(tok >> 4) * G;
     const int m = tok & 15;
     const bool live = tok < T;                             // the last tile's other tokens are zero
     const float* xr = x + (size_t)min(tok, T - 1) * H;
-    const float inv_rms = rms_inv_256(xr, H, eps, red);
-    for (int c = t; c < H / 8; c += 256) {                 // H / 8 is a multiple of 4: a group's lanes stay together
-        const float4* p = reinterpret_cast<const float4*>(xr + 8 * c);
-        const float4 p0 = p[0], p1 = p[1];
-        const uint4 w4 = *reinterpret_cast<const uint4*>(nw + 8 * c);
-        const uint32_t w[4] = {w4.x, w4.y, w4.z, w4.w};
-        float v[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+    float4 p[NC][2];
+    uint4 w4[NC];
+    auto load = [&](int k, int c) {
+        const float4* s = reinterpret_cast<const float4*>(xr + 8 * c);
+        p[k][0] = s[0];
+        p[k][1] = s[1];
+        w4[k] = *reinterpret_cast<const uint4*>(nw + 8 * c);
+    };
+    float inv_rms;
+    if constexpr (KU > 0) {
+        float xs[KU];
+#pragma unroll
+        for (int i = 0; i < KU; i++) xs[i] = xr[t + 256 * i];
+#pragma unroll
+        for (int k = 0; k < NC; k++) load(k, min(t + 256 * k, H / 8 - 1));
+        TI_ISSUE_FENCE();
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < KU; i++) {
+            const float sq = xs[i] * xs[i];
+            s = s + sq;
+        }
+        float mean = ti_tree_sum_256(s, red) / (float)H;
+        mean = mean + eps;
+        inv_rms = 1.0f / sqrtf(mean);
+    } else {
+        inv_rms = rms_inv_256(xr, H, eps, red);
+    }
+    auto chunk = [&](int k, int c) {
+        const uint32_t w[4] = {w4[k].x, w4[k].y, w4[k].z, w4[k].w};
+        float v[8] = {p[k][0].x, p[k][0].y, p[k][0].z, p[k][0].w, p[k][1].x, p[k][1].y, p[k][1].z, p[k][1].w};
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const float n = v[i] * inv_rms;
@@ -332,6 +360,17 @@ __global__ __launch_bounds__(256) void k_norm_frag(const float* __restrict__ x, 
         const int g = c >> 2, j = c & 3;
         xh[(f0 + g) * 64 + 16 * j + m] = h;
         if (j == 0) xsc[(f0 + g) * 16 + m] = scale;
+    };
+    // H / 8 is a multiple of 4: a group's four lanes stay together
+    if constexpr (KU > 0) {
+#pragma unroll
+        for (int k = 0; k < NC; k++)
+            if (t + 256 * k < H / 8) chunk(k, t + 256 * k);
+    } else {
+        for (int c = t; c < H / 8; c += 256) {
+            load(0, c);
+            chunk(0, c);
+        }
     }
 }
 
@@ -398,7 +437,11 @@ int ti_quant_frag_launch(ti_ctx* c, const float* x, const TiFrag& f, int T, int 
 }
 
 int ti_norm_frag_launch(ti_ctx* c, const float* x, const uint16_t* w, float eps, const TiFrag& f, int T, int H) {
-    k_norm_frag<<<(unsigned)((T + 15) / 16 * 16), 256, 0, c->stream>>>(x, w, eps, reinterpret_cast<ti_h8*>(f.xh), f.sc, T, H);
+    const unsigned grid = (unsigned)((T + 15) / 16 * 16);
+    ti_h8* xh = reinterpret_cast<ti_h8*>(f.xh);
+    if (H == 1024) k_norm_frag<4><<<grid, 256, 0, c->stream>>>(x, w, eps, xh, f.sc, T, H);
+    else if (H == 2048) k_norm_frag<8><<<grid, 256, 0, c->stream>>>(x, w, eps, xh, f.sc, T, H);
+    else k_norm_frag<0><<<grid, 256, 0, c->stream>>>(x, w, eps, xh, f.sc, T, H);
     TI_LAUNCHED("k_norm_frag");
     return TI_OK;
 }

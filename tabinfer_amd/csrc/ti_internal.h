@@ -149,6 +149,9 @@ int ti_tgemm_launch(ti_ctx* c, const TgIn& in, int nseg, const uint32_t* const* 
                     float* const* ys, const int* Ns, int T, int K, int acc, float* pout);
 int ti_tgemm_gateup_launch(ti_ctx* c, const TgIn& in, const uint32_t* gpack, const uint16_t* gsc, const uint32_t* upack,
                            const uint16_t* usc, int I, int H, int T, uint32_t* swq, float* sws);
+int ti_pattn_prep_launch(ti_ctx* c, const float* q, const float* k, const float* v, const uint16_t* qw, const uint16_t* kw,
+                         const float* rope, float eps, float* qr, uint32_t* kq, float* ks, uint32_t* vq, float* vs, int pos,
+                         int T, int nHq, int nKv, int kvs);
 bool ti_pattn_ok(int T, int nHq, int nKv, int hd);
 int ti_pattn_launch(ti_ctx* c, const float* qr, const uint32_t* kq, const float* ks, const uint32_t* vq, const float* vs,
                     float* out, const TiFrag* frag, int S0, int T, int nHq, int nKv, int kvs);

@@ -119,11 +119,6 @@ __global__ void k_swiglu(const float* __restrict__ g, const float* __restrict__ 
     if (i < n) { float a = g[i]; y[i] = a / (1.0f + expf(-a)) * u[i]; }
 }
 
-__global__ void k_copy_f32(const float* __restrict__ s, float* __restrict__ d, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) d[i] = s[i];
-}
-
 // ---------------------------------------------------------------------------
 // model
 // ---------------------------------------------------------------------------
@@ -147,7 +142,7 @@ struct ti_qwen3 {
     uint16_t* embed = nullptr;
     uint16_t* final_norm = nullptr;
     Lin lm;
-    float *x, *normed, *q, *k, *v, *qr, *kr, *attn, *gate, *up, *swi, *last, *logits;
+    float *x, *normed, *q, *k, *v, *qr, *kr, *attn, *gate, *up, *swi, *logits;
     uint32_t* xq;
     float* xs;
     int32_t* xsum;
@@ -293,7 +288,7 @@ extern "C" int ti_qwen3_create(ti_ctx* c, const ti_qwen3_config* cfg, ti_qwen3**
     struct { float** p; size_t n; } fb[] = {{&m->x, (size_t)T * H}, {&m->normed, (size_t)T * H}, {&m->q, (size_t)T * nq},
                                             {&m->k, (size_t)T * nkv}, {&m->v, (size_t)T * nkv}, {&m->qr, (size_t)T * nq},
                                             {&m->kr, (size_t)T * nkv}, {&m->attn, (size_t)T * nq}, {&m->gate, (size_t)T * I},
-                                            {&m->up, (size_t)T * I}, {&m->swi, (size_t)T * I}, {&m->last, (size_t)H},
+                                            {&m->up, (size_t)T * I}, {&m->swi, (size_t)T * I},
                                             {&m->logits, (size_t)C.vocab}, {&m->amx_v, (size_t)AMX_PARTS}};
     for (auto& f : fb) if (!rc) rc = mk(m, (void**)f.p, f.n * 4);
     const size_t kmax = (size_t)(H > I ? (H > nq ? H : nq) : (I > nq ? I : nq));   // widest GEMV input
@@ -634,7 +629,7 @@ extern "C" int ti_qwen3_forward(ti_ctx* c, ti_qwen3* m, const int32_t* ids, int 
     const bool fused_attn = ti_tattn_ok(T, nHq, nKv, hd);
     const bool norm_in = fused && T <= 4 && ti_tgemm_norm_ok(T, H);
     // Longer prompts (and widths without a short-batch kernel): [rmsnorm + quantQ8T] [q/k/v]
-    // [attention] [merge + quantQ8T] [o_proj + residual] [rmsnorm + quantQ8T]
+    // [rotary + KV write] [attention] [merge + quantQ8T] [o_proj + residual] [rmsnorm + quantQ8T]
     // [gate/up + SiLU + quantQ8T] [down + residual] (k_gemm.hip, k_pattn.hip). A traced forward, whose fields hold the
     // f32 SwiGLU, and a single token outside a decode step run operation by operation.
     const bool prompt = !fused && T > 1 && !m->trace && ti_gemm_ok(H) && ti_gemm_ok(nq) && ti_gemm_ok(I);
@@ -675,15 +670,16 @@ extern "C" int ti_qwen3_forward(ti_ctx* c, ti_qwen3* m, const int32_t* ids, int 
         if (fused && fused_attn) {
             RC(ti_tattn_launch(c, m->q, m->k, m->v, y.q_norm, y.k_norm, m->rope, y.kq, y.ks, y.vq, y.vs, pos, T, nHq, nKv,
                                hd, C.rms_eps, m->xq, m->xs, m->kvs));
+        } else if (pattn) {
+            RC(ti_pattn_prep_launch(c, m->q, m->k, m->v, y.q_norm, y.k_norm, m->rope, C.rms_eps, m->qr, y.kq, y.ks, y.vq, y.vs,
+                                    pos, T, nHq, nKv, m->kvs));
+            RC(ti_pattn_launch(c, m->qr, y.kq, y.ks, y.vq, y.vs, nullptr, &cfrag, pos + 1, T, nHq, nKv, m->kvs));
         } else {
             RC(ti_rope_qk(c, m->q, y.q_norm, m->qr, T, nHq, hd, pos, C.rope_theta, C.rms_eps));
             RC(ti_rope_qk(c, m->k, y.k_norm, m->kr, T, nKv, hd, pos, C.rope_theta, C.rms_eps));
             RC(ti_kv_write_launch(c, m->kr, m->v, y.kq, y.ks, y.vq, y.vs, T, nKv, hd, pos, m->kvs));
-            if (pattn)
-                RC(ti_pattn_launch(c, m->qr, y.kq, y.ks, y.vq, y.vs, nullptr, &cfrag, pos + 1, T, nHq, nKv, m->kvs));
-            else
-                RC(ti_attn_decode_launch(c, m->qr, y.kq, y.ks, y.vq, y.vs, m->attn, pos + 1, T, nHq, nKv, hd, 0, nullptr, 0,
-                                         m->kvs));
+            RC(ti_attn_decode_launch(c, m->qr, y.kq, y.ks, y.vq, y.vs, m->attn, pos + 1, T, nHq, nKv, hd, 0, nullptr, 0,
+                                     m->kvs));
         }
         RC(trace_put(c, m, l, TR_Q, m->q, T));
         RC(trace_put(c, m, l, TR_K, m->k, T));
@@ -726,10 +722,8 @@ extern "C" int ti_qwen3_forward(ti_ctx* c, ti_qwen3* m, const int32_t* ids, int 
         RC(ti_linear_q4(c, m->swi, y.down.pack, y.down.sc, m->x, T, H, I, 1));
     }
     RC(trace_put(c, m, C.layers, TR_X_IN, m->x, T));
-    k_copy_f32<<<(H + 255) / 256, 256, 0, c->stream>>>(m->x + (size_t)(T - 1) * H, m->last, H);
-    TI_LAUNCHED("k_copy_f32");
-    RC(ti_fused_lmhead_launch(c, m->last, m->final_norm, C.rms_eps, m->lm.pack, m->lm.sc, m->logits, C.vocab, H, m->hist,
-                              nullptr, pos + T, C.max_ctx, nullptr, nullptr, 0, m->samp));
+    RC(ti_fused_lmhead_launch(c, m->x + (size_t)(T - 1) * H, m->final_norm, C.rms_eps, m->lm.pack, m->lm.sc, m->logits, C.vocab,
+                              H, m->hist, nullptr, pos + T, C.max_ctx, nullptr, nullptr, 0, m->samp));
     k_set_pos<<<1, 256, 0, c->stream>>>(m->dpos, pos + T, m->rope, m->rope_cur, hd, C.max_ctx);
     TI_LAUNCHED("k_set_pos");
     m->pos_hint = pos + T < C.max_ctx ? pos + T : C.max_ctx - 1;
