@@ -347,8 +347,8 @@ __global__ __launch_bounds__(ATT_THREADS) void k_attn_split_q8(const float* __re
 }
 
 // ---------------------------------------------------------------------------
-// T > 1 queries (a prefill chunk or a T-token batch, models/qwen3.js:2534-2577): one
-// pass over a split's keys serves every query row of the KV head, instead of one pass
+// T > 1 queries of at most 32 rows a KV head (a T-token batch, models/qwen3.js:2534-2577; more take
+// k_pattn.hip): one pass over a split's keys serves every query row of the KV head, instead of one pass
 // per query. Workgroup (256 threads) = (split, KV head, group of 16 query rows; row
 // ri = (t, h) with t = query, h = head of the group). Key tiles of 64:
 //  - S = Q K^T on the matrix cores: v_mfma_f32_16x16x32_f16, one MFMA per 32-dim scale
