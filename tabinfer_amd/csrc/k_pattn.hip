@@ -3,33 +3,35 @@
 //
 // Workgroup (4 waves): one KV head, one range of keys, 64 query rows (row = token x query head of the
 // KV head); a wave owns 16 rows and meets the others only over the staged keys. Key blocks of 64 are
-// staged in LDS as MFMA operands (f16 codes, exact), the next block's loads in flight meanwhile.
+// staged in LDS as MFMA operands (K codes f16, V codes bf16, exact), the next block's loads in flight meanwhile.
 //   - S^T = K Q^T, one v_mfma_f32_16x16x32_f16 per 32-dim scale group, 16 keys and q half: q = hi + lo in
 //     f16 (to 2^-22), each group's sum scaled by its key's scale in f32. Transposed, a lane's scores are
 //     those of one query row, keys 4j..4j+3 of each 16: the P operand of the second product as they
 //     stand, and the row's running maximum and sum live in its own four lanes.
-//   - O^T = V^T P^T with P times the V scale of (key, group), again split into f16 hi + lo. The scales
-//     are taken relative to the power of two under the range's largest of that group, and 2^10 up, so
-//     that hi lies in f16's normal range and what hi + lo lose is 2^-36 of the largest weight.
+//   - O^T = V^T P^T with P times the V scale of (key, group) in f32, split into three bf16, exactly: bf16 has
+//     f32's exponents, so a weight is as exact as in f32 beside any other, and what one key's scale is does not
+//     touch another's. (Two f16 under a common power of two take 5% less time, but lose all of a weight
+//     2^-36 of the largest scale of its keys.) The codes are exact in bf16.
 // What bounds it is latency first (a workgroup has 2 to 4 blocks; its loads of q are issued before all
 // else, and three workgroups share a CU), then the VALU work of the weights (scale, mask, exponential,
-// four scaled splits). With 32 rows a wave, whose operands are read from LDS for two products, only two
+// four scaled three-fold splits). With 32 rows a wave, whose operands are read from LDS for two products, only two
 // fit: 256 tokens at 3840 47.7 against 46.7 us, at 0 26 against 15.
 // The ranges' partials (o, m, l; m in log2) are merged by k_pattn_merge, which also quantizes the output
 // into the o projection's fragments (k_gemm.hip) when asked.
-// 256 tokens x 16 heads over 4096 keys: 48.5 us with the merge, against 353 of k_attn_multi_q8 (P V as f32
-// FMAs, a workgroup per 16 rows); error against 64 bits 2.3e-7, against 2.5e-7.
+// 256 tokens x 16 heads over 4096 keys: 51.3 us with the merge, against 353 of k_attn_multi_q8 (P V as f32
+// FMAs, a workgroup per 16 rows); error against 64 bits 2.4e-7, against 2.5e-7.
 #include "ti_dev.h"
 
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));   // the caller's q need not be aligned
 
 constexpr int HD = 128, NG = HD / 32, KB = 64;         // KB: keys of a staged block
 constexpr int VSTRIDE = 65;                            // 16-byte pieces of a V operand tile (1 of padding: writes of
                                                        // eight tiles would meet in one bank)
-constexpr uint32_t WUP = 10;                           // log2 of the weights' factor
 constexpr float MLOW = -3.0e38f;
 
 struct PattnArgs {
@@ -46,9 +48,8 @@ struct PattnArgs {
 
 struct PattnLds {
     ti_h8 k[KB / 16][NG][64];                          // [16 keys][group][lane]: key lane % 16, dims 8 (lane / 16)..
-    ti_h8 v[KB / 32][8][VSTRIDE];                      // [32 keys][16 dims][lane]: dim lane % 16, keys 4j.., 16 + 4j..
+    v8bf v[KB / 32][8][VSTRIDE];                       // [32 keys][16 dims][lane]: dim lane % 16, keys 4j.., 16 + 4j..
     float ks[NG][KB], vs[NG][KB];
-    float vmax[4][NG];
 };
 
 // 4 x 4 bytes: in, w[r] = row r's four bytes; out, w[e] = byte e of rows 0..3
@@ -61,6 +62,28 @@ __device__ __forceinline__ void tr4_bytes(uint32_t (&w)[4]) {
     w[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
     w[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
     w[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
+}
+
+// four int8 -> bf16, exact
+__device__ __forceinline__ uint2 i8x4_bf16(uint32_t w) {
+    float f[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) f[i] = (float)(int8_t)(w >> (8 * i));
+    return make_uint2(__builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f[1]), __builtin_bit_cast(uint32_t, f[0]), 0x07060302u),
+                      __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f[3]), __builtin_bit_cast(uint32_t, f[2]), 0x07060302u));
+}
+
+// A f32 as the sum of three bf16, exactly: its top 8 bits, the top 8 of what is left, the rest.
+// bf16_tops: the top halves of two floats, side by side; bf16_rest: v less the half of `tops` that sel
+// names with -1 (the other with 0)
+__device__ __forceinline__ uint32_t bf16_tops(float a, float b) {
+    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+}
+__device__ __forceinline__ float bf16_rest(uint32_t tops, uint32_t sel, float v) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, tops), __builtin_bit_cast(v2bf, sel), v, false);
+}
+__device__ __forceinline__ v8bf bf16_op(const uint32_t (&w)[4]) {
+    return __builtin_bit_cast(v8bf, make_uint4(w[0], w[1], w[2], w[3]));
 }
 
 __global__ __launch_bounds__(256, 3) void k_pattn(PattnArgs a) {
@@ -113,23 +136,10 @@ __global__ __launch_bounds__(256, 3) void k_pattn(PattnArgs a) {
     }
     if (c0 < c1) load(c0);
 
-    // the range's largest V scale of each group -> the power of two under it
-    float gmax = 0.0f;
-    for (int t = c0 + (tid >> 2); t < c1; t += 64) gmax = fmaxf(gmax, vsp[t * scale_row + (tid & 3)]);
-#pragma unroll
-    for (int o = 4; o < 64; o <<= 1) gmax = fmaxf(gmax, ti_xor(gmax, o));
-    if (lane < NG) L.vmax[wave][lane] = gmax;
-    __syncthreads();
-    auto pow2 = [&](int g) {
-        const float v = fmaxf(fmaxf(L.vmax[0][g], L.vmax[1][g]), fmaxf(L.vmax[2][g], L.vmax[3][g]));
-        const uint32_t e = __builtin_bit_cast(uint32_t, v) & 0x7f800000u;
-        return min(max(e, 0x08000000u), 0x7e000000u);
-    };
-    // 2^(WUP - e) for the group this thread stages
-    const float vdown = __builtin_bit_cast(float, 0x7f000000u - pow2(tid & 3) + (WUP << 23));
-
-    float neg = -1.0f;                                     // opaque: w - hi as one v_fma_mix, not convert and subtract
+    float neg = -1.0f;                                     // opaque: q - hi as one v_fma_mix, not convert and subtract
     asm("" : "+s"(neg));
+    uint32_t even = 0x0000BF80u, odd = 0xBF800000u;        // (-1, 0) and (0, -1): bf16_rest
+    asm("" : "+s"(even), "+s"(odd));
     // Q operand: dims 32 g + 8 j.., hi and lo; and the keys the row sees
     ti_h8 qh[NG], ql[NG];
 #pragma unroll
@@ -161,14 +171,12 @@ __global__ __launch_bounds__(256, 3) void k_pattn(PattnArgs a) {
             tr4_bytes(vr[u]);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                ti_h2 h0, h1;
-                ti_i8x4_h2x2(vr[u][e], h0, h1);
-                ti_h8* p = &L.v[kb >> 3][vdb >> 2][(kk & 3) * 16 + 4 * (vdb & 3) + e];
-                reinterpret_cast<uint2*>(p)[kk >> 2] = make_uint2(__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1));
+                v8bf* p = &L.v[kb >> 3][vdb >> 2][(kk & 3) * 16 + 4 * (vdb & 3) + e];
+                reinterpret_cast<uint2*>(p)[kk >> 2] = i8x4_bf16(vr[u][e]);
             }
         }
         L.ks[tid & 3][tid >> 2] = ksr;
-        L.vs[tid & 3][tid >> 2] = vsr * vdown;
+        L.vs[tid & 3][tid >> 2] = vsr;
         __syncthreads();
         if (t0 + KB < c1) load(t0 + KB);
         TI_ISSUE_FENCE();
@@ -223,25 +231,23 @@ __global__ __launch_bounds__(256, 3) void k_pattn(PattnArgs a) {
             for (int g = 0; g < NG; g++) {
                 const v4f v0 = *reinterpret_cast<const v4f*>(&L.vs[g][32 * h + 4 * j]);
                 const v4f v1 = *reinterpret_cast<const v4f*>(&L.vs[g][32 * h + 16 + 4 * j]);
-                ti_h8 ph, pl;
+                uint32_t w0[4], w1[4], w2[4];
 #pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    const float w0 = e < 4 ? s[0][e] * v0[e] : s[1][e - 4] * v1[e - 4];
-                    const float w1 = e < 4 ? s[0][e + 1] * v0[e + 1] : s[1][e - 3] * v1[e - 3];
-                    // opaque: else lo may be taken from a hi that was rounded from the unrounded product
-                    uint32_t hp = __builtin_bit_cast(uint32_t, ti_h2{(_Float16)w0, (_Float16)w1});
-                    asm("" : "+v"(hp));
-                    const ti_h2 hi = __builtin_bit_cast(ti_h2, hp);
-                    ph[e] = hi[0];
-                    ph[e + 1] = hi[1];
-                    pl[e] = (_Float16)fmaf((float)hi[0], neg, w0);
-                    pl[e + 1] = (_Float16)fmaf((float)hi[1], neg, w1);
+                for (int k = 0; k < 4; k++) {              // keys 2k, 2k + 1 of the lane's eight
+                    const float a0 = s[k / 2][2 * (k % 2)] * (k < 2 ? v0 : v1)[2 * (k % 2)];
+                    const float a1 = s[k / 2][2 * (k % 2) + 1] * (k < 2 ? v0 : v1)[2 * (k % 2) + 1];
+                    w0[k] = bf16_tops(a0, a1);
+                    const float b0 = bf16_rest(w0[k], even, a0), b1 = bf16_rest(w0[k], odd, a1);
+                    w1[k] = bf16_tops(b0, b1);
+                    w2[k] = bf16_tops(bf16_rest(w1[k], even, b0), bf16_rest(w1[k], odd, b1));
                 }
+                const v8bf p0 = bf16_op(w0), p1 = bf16_op(w1), p2 = bf16_op(w2);
 #pragma unroll
                 for (int d = 2 * g; d < 2 * g + 2; d++) {
-                    const ti_h8 vv = L.v[h][d][lane];
-                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, ph, o[d], 0, 0, 0);
-                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, pl, o[d], 0, 0, 0);
+                    const v8bf vv = L.v[h][d][lane];
+                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p2, o[d], 0, 0, 0);
+                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p1, o[d], 0, 0, 0);
+                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p0, o[d], 0, 0, 0);
                 }
             }
         }
@@ -252,7 +258,7 @@ __global__ __launch_bounds__(256, 3) void k_pattn(PattnArgs a) {
     const size_t slot = ((size_t)tok * a.nHq + hq) * a.nsplit + split;
 #pragma unroll
     for (int d = 0; d < 8; d++)
-        *reinterpret_cast<v4f*>(a.po + slot * HD + 16 * d + 4 * j) = o[d] * __builtin_bit_cast(float, pow2(d / 2) - (WUP << 23));
+        *reinterpret_cast<v4f*>(a.po + slot * HD + 16 * d + 4 * j) = o[d];
     if (j == 0) {
         a.pml[2 * slot] = mx;
         a.pml[2 * slot + 1] = l;
