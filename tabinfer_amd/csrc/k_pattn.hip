@@ -25,8 +25,6 @@
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));   // the caller's q need not be aligned
 
 constexpr int HD = 128, NG = HD / 32, KB = 64;         // KB: keys of a staged block
@@ -48,7 +46,7 @@ struct PattnArgs {
 
 struct PattnLds {
     ti_h8 k[KB / 16][NG][64];                          // [16 keys][group][lane]: key lane % 16, dims 8 (lane / 16)..
-    v8bf v[KB / 32][8][VSTRIDE];                       // [32 keys][16 dims][lane]: dim lane % 16, keys 4j.., 16 + 4j..
+    ti_b8 v[KB / 32][8][VSTRIDE];                       // [32 keys][16 dims][lane]: dim lane % 16, keys 4j.., 16 + 4j..
     float ks[NG][KB], vs[NG][KB];
 };
 
@@ -62,28 +60,6 @@ __device__ __forceinline__ void tr4_bytes(uint32_t (&w)[4]) {
     w[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
     w[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
     w[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
-}
-
-// four int8 -> bf16, exact
-__device__ __forceinline__ uint2 i8x4_bf16(uint32_t w) {
-    float f[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) f[i] = (float)(int8_t)(w >> (8 * i));
-    return make_uint2(__builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f[1]), __builtin_bit_cast(uint32_t, f[0]), 0x07060302u),
-                      __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f[3]), __builtin_bit_cast(uint32_t, f[2]), 0x07060302u));
-}
-
-// A f32 as the sum of three bf16, exactly: its top 8 bits, the top 8 of what is left, the rest.
-// bf16_tops: the top halves of two floats, side by side; bf16_rest: v less the half of `tops` that sel
-// names with -1 (the other with 0)
-__device__ __forceinline__ uint32_t bf16_tops(float a, float b) {
-    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
-}
-__device__ __forceinline__ float bf16_rest(uint32_t tops, uint32_t sel, float v) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, tops), __builtin_bit_cast(v2bf, sel), v, false);
-}
-__device__ __forceinline__ v8bf bf16_op(const uint32_t (&w)[4]) {
-    return __builtin_bit_cast(v8bf, make_uint4(w[0], w[1], w[2], w[3]));
 }
 
 __global__ __launch_bounds__(256, 3) void k_pattn(PattnArgs a) {
@@ -138,8 +114,6 @@ __global__ __launch_bounds__(256, 3) void k_pattn(PattnArgs a) {
 
     float neg = -1.0f;                                     // opaque: q - hi as one v_fma_mix, not convert and subtract
     asm("" : "+s"(neg));
-    uint32_t even = 0x0000BF80u, odd = 0xBF800000u;        // (-1, 0) and (0, -1): bf16_rest
-    asm("" : "+s"(even), "+s"(odd));
     // Q operand: dims 32 g + 8 j.., hi and lo; and the keys the row sees
     ti_h8 qh[NG], ql[NG];
 #pragma unroll
@@ -171,8 +145,8 @@ __global__ __launch_bounds__(256, 3) void k_pattn(PattnArgs a) {
             tr4_bytes(vr[u]);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                v8bf* p = &L.v[kb >> 3][vdb >> 2][(kk & 3) * 16 + 4 * (vdb & 3) + e];
-                reinterpret_cast<uint2*>(p)[kk >> 2] = i8x4_bf16(vr[u][e]);
+                ti_b8* p = &L.v[kb >> 3][vdb >> 2][(kk & 3) * 16 + 4 * (vdb & 3) + e];
+                reinterpret_cast<uint2*>(p)[kk >> 2] = ti_i8x4_b4(vr[u][e]);
             }
         }
         L.ks[tid & 3][tid >> 2] = ksr;
@@ -231,23 +205,19 @@ __global__ __launch_bounds__(256, 3) void k_pattn(PattnArgs a) {
             for (int g = 0; g < NG; g++) {
                 const v4f v0 = *reinterpret_cast<const v4f*>(&L.vs[g][32 * h + 4 * j]);
                 const v4f v1 = *reinterpret_cast<const v4f*>(&L.vs[g][32 * h + 16 + 4 * j]);
-                uint32_t w0[4], w1[4], w2[4];
+                float w[8];
 #pragma unroll
-                for (int k = 0; k < 4; k++) {              // keys 2k, 2k + 1 of the lane's eight
-                    const float a0 = s[k / 2][2 * (k % 2)] * (k < 2 ? v0 : v1)[2 * (k % 2)];
-                    const float a1 = s[k / 2][2 * (k % 2) + 1] * (k < 2 ? v0 : v1)[2 * (k % 2) + 1];
-                    w0[k] = bf16_tops(a0, a1);
-                    const float b0 = bf16_rest(w0[k], even, a0), b1 = bf16_rest(w0[k], odd, a1);
-                    w1[k] = bf16_tops(b0, b1);
-                    w2[k] = bf16_tops(bf16_rest(w1[k], even, b0), bf16_rest(w1[k], odd, b1));
+                for (int e = 0; e < 4; e++) {
+                    w[e] = s[0][e] * v0[e];
+                    w[4 + e] = s[1][e] * v1[e];
                 }
-                const v8bf p0 = bf16_op(w0), p1 = bf16_op(w1), p2 = bf16_op(w2);
+                ti_b8 p[3];
+                ti_bf16x3(w, p);
 #pragma unroll
                 for (int d = 2 * g; d < 2 * g + 2; d++) {
-                    const v8bf vv = L.v[h][d][lane];
-                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p2, o[d], 0, 0, 0);
-                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p1, o[d], 0, 0, 0);
-                    o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p0, o[d], 0, 0, 0);
+                    const ti_b8 vv = L.v[h][d][lane];
+#pragma unroll
+                    for (int i = 2; i >= 0; i--) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, p[i], o[d], 0, 0, 0);
                 }
             }
         }

@@ -21,7 +21,8 @@
 //  - P V on the matrix cores as well: the scores come out of the MFMA with lane (r, j)
 //    holding row r at keys 4j..4j+3 of each 16-key half, which is already the A-operand
 //    layout of the next MFMA (K index 8j + e <-> key 4j + e, 16 + 4j + e - 4); the V
-//    scale of (key, 32-dim group) is folded into P (P'_g = p * vs, again f16 hi + lo);
+//    scale of (key, 32-dim group) is folded into P (P'_g = p * vs in f32, as three bf16, exactly:
+//    any scale, and no 16-bit rounding of its own);
 //    the V operand (8 keys of one dim per lane) comes from the key-major V tile through
 //    gfx950's transposing LDS read ds_read_b64_tr_b8 (16 lanes read 8 rows of 16 bytes,
 //    lane i receives column i), whose row addresses follow the same key order;
@@ -304,8 +305,8 @@ __global__ __launch_bounds__(64 * TA_W) void k_attn_tq8(TAttnArgs a) {
         }
         // online softmax of row r16 (its 32 keys sit in lanes r16 + 16j), base 2. The
         // reference maximum moves only when the block's maximum exceeds it by more than 6
-        // (p <= 64, far inside f16 for p * vs), so O is rescaled rarely; the result is
-        // unchanged (o and l share the reference)
+        // (p <= 64), so O is rescaled rarely; the result is unchanged (o and l share the
+        // reference)
         float mt = sc[0][0];
 #pragma unroll
         for (int b = 0; b < 2; b++)
@@ -335,8 +336,8 @@ __global__ __launch_bounds__(64 * TA_W) void k_attn_tq8(TAttnArgs a) {
                 for (int D = 0; D < 8; D++) O[D][i] *= ci;
             }
         }
-        // P'_g = p * vs(key, g) as f16 hi + lo, A operands: K index 8jq + 4b + i
-        h8 ph[NG], pl[NG];
+        // P'_g = p * vs(key, g) as three bf16, A operands: K index 8jq + 4b + i
+        float pv[NG][8];
 #pragma unroll
         for (int b = 0; b < 2; b++)
 #pragma unroll
@@ -344,12 +345,7 @@ __global__ __launch_bounds__(64 * TA_W) void k_attn_tq8(TAttnArgs a) {
                 const float4 vg = *reinterpret_cast<const float4*>(&s_vs[reg][16 * b + 4 * jq + i][0]);
                 const float vv[4] = {vg.x, vg.y, vg.z, vg.w};
 #pragma unroll
-                for (int g = 0; g < NG; g++) {
-                    const float pv = p[b][i] * vv[g];
-                    const _Float16 hi = (_Float16)pv;
-                    ph[g][4 * b + i] = hi;
-                    pl[g][4 * b + i] = (_Float16)(pv - (float)hi);
-                }
+                for (int g = 0; g < NG; g++) pv[g][4 * b + i] = p[b][i] * vv[g];
             }
         // V operands through the transposing read: lanes 2rr, 2rr+1 of a 16-lane group
         // address key(8jq + rr) (rr < 4: 4jq + rr; else 16 + 4jq + rr - 4), 8-byte halves
@@ -358,12 +354,18 @@ __global__ __launch_bounds__(64 * TA_W) void k_attn_tq8(TAttnArgs a) {
         const int kv_row = rr < 4 ? 4 * jq + rr : 16 + 4 * jq + (rr - 4);
         const uint8_t* vrow = vt + kv_row * TA_VS + 8 * (r16 & 1);
 #pragma unroll
-        for (int D = 0; D < 8; D++) {
-            const v2i vb = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-                (__attribute__((address_space(3))) v2i*)(vrow + 16 * D));
-            const h8 vh = ti_i8x8_h8((uint32_t)vb.x, (uint32_t)vb.y);
-            O[D] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[D >> 1], vh, O[D], 0, 0, 0);
-            O[D] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl[D >> 1], vh, O[D], 0, 0, 0);
+        for (int g = 0; g < NG; g++) {
+            ti_b8 pb[3];
+            ti_bf16x3(pv[g], pb);
+#pragma unroll
+            for (int D = 2 * g; D < 2 * g + 2; D++) {
+                const v2i vb = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                    (__attribute__((address_space(3))) v2i*)(vrow + 16 * D));
+                const uint2 lo = ti_i8x4_b4((uint32_t)vb.x), hi = ti_i8x4_b4((uint32_t)vb.y);
+                const ti_b8 vh = __builtin_bit_cast(ti_b8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+#pragma unroll
+                for (int i = 2; i >= 0; i--) O[D] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pb[i], vh, O[D], 0, 0, 0);
+            }
         }
     };
 

@@ -196,6 +196,40 @@ __device__ __forceinline__ ti_h8 ti_i8x8_h8(uint32_t lo, uint32_t hi) {
     return __builtin_bit_cast(ti_h8, w);
 }
 
+__device__ __forceinline__ uint32_t ti_bf16_tops(float a, float b) {   // the top halves of two floats, side by side
+    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+}
+// four int8 -> bf16, exactly
+__device__ __forceinline__ uint2 ti_i8x4_b4(uint32_t w) {
+    return make_uint2(ti_bf16_tops((float)(int8_t)w, (float)(int8_t)(w >> 8)),
+                      ti_bf16_tops((float)(int8_t)(w >> 16), (float)(int8_t)(w >> 24)));
+}
+
+// Eight f32 as three MFMA operands of bf16 whose sum they are, exactly (bf16 has f32's exponents): the top 8
+// bits of each, the top 8 of what is left, the rest. What is left of one of a pair is one
+// v_dot2_f32_bf16 of the pair's tops and (-1, 0) or (0, -1); 3.5 operations a value.
+typedef __bf16 ti_b2 __attribute__((ext_vector_type(2)));
+typedef __bf16 ti_b8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ void ti_bf16x3(const float (&v)[8], ti_b8 (&op)[3]) {
+    uint32_t even = 0x0000BF80u, odd = 0xBF800000u;
+    asm("" : "+s"(even), "+s"(odd));
+    const ti_b2 se = __builtin_bit_cast(ti_b2, even), so = __builtin_bit_cast(ti_b2, odd);
+    uint32_t w[3][4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        float a = v[2 * k], b = v[2 * k + 1];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            w[i][k] = ti_bf16_tops(a, b);
+            if (i == 2) break;
+            a = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(ti_b2, w[i][k]), se, a, false);
+            b = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(ti_b2, w[i][k]), so, b, false);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) op[i] = __builtin_bit_cast(ti_b8, make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]));
+}
+
 // Keep every memory operation issued so far above this point: the scheduler may
 // otherwise sink a kernel's weight loads below the wait for its activation loads,
 // which serialises two memory round trips that were meant to overlap.
