@@ -232,11 +232,13 @@ __global__ __launch_bounds__(256, 2) void k_bb_attn(const float* __restrict__ qr
     v4f o[8] = {};                                     // tile (h, e): dims 64 h + 4 c + e, c = 4 j + i in element i
     if (k0 + wave < k1) load(k0 + wave);
     for (int tile = k0 + wave; tile < k1; tile += 4) {
+        ti_wave_lds_fence();                           // the last tile is read
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             L.k[2 * i + lr][lp] = kr[i];
             L.v[2 * i + lr][lp] = vr[i];
         }
+        ti_wave_lds_fence();
         if (tile + 4 < k1) load(tile + 4);
         v4f s = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll

@@ -61,13 +61,6 @@ __device__ __forceinline__ void tr4_rows(const uint4 w, uint32_t (&b)[4]) {
     b[3] = r1[1];
 }
 
-// one wave's LDS reads follow its own LDS writes without a barrier (the unit serves a wave in
-// order); this keeps the compiler from moving either across
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // GU: tiles 0, 1 are gate rows +0 / +16 of the workgroup's 32-row chunk, 2, 3 the same up rows
 template <bool GU, int NT, int MT, int W>
 __global__ __launch_bounds__(64 * W, 2) void k_gemm_q4(GemmArgs a) {
@@ -141,7 +134,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_gemm_q4(GemmArgs a) {
     load_a(A[0], 4 * wave);
     for (int st = wave; 4 * st < G; st += W) {
         uint32_t bw[NT][4];
-        wave_lds_fence();                                  // the last step's reads are done
+        ti_wave_lds_fence();                                  // the last step's reads are done
 #pragma unroll
         for (int n = 0; n < NT; n++) {
             L.sw[n][j][m] = 4 * st + j < G ? ti_h2f(sw[n]) : 0.0f;
@@ -149,7 +142,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_gemm_q4(GemmArgs a) {
         }
 #pragma unroll
         for (int t = 0; t < MT; t++) L.sx[t][j][m] = sx[t];
-        wave_lds_fence();
+        ti_wave_lds_fence();
         load_step(st + W);
         TI_ISSUE_FENCE();
 #pragma unroll

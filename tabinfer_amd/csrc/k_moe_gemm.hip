@@ -65,11 +65,6 @@ __device__ __forceinline__ ti_h8 q3_f16(uint32_t x) {
     return __builtin_bit_cast(ti_h8, w);
 }
 
-__device__ __forceinline__ void wave_lds_fence() {         // one wave's LDS reads behind its own writes
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 constexpr int SCAN = 1024;         // routing ids listed at a time: a second list would read the weights again
 constexpr int MTX = 2;             // 16-pair tiles of one pass, at most
 
@@ -135,7 +130,7 @@ __device__ __forceinline__ void moe_sums(const MoeGemm& a, const MoeRows<NT>& ro
     for (int st = wave; 4 * st < G; st += W) {
         uint32_t nib[NT][4];
         v4f sum[NT][MT];
-        wave_lds_fence();                                  // the last step's reads are done
+        ti_wave_lds_fence();                                  // the last step's reads are done
 #pragma unroll
         for (int t = 0; t < MT; t++) L.sx[t][j][m] = xn[t];
 #pragma unroll
@@ -145,7 +140,7 @@ __device__ __forceinline__ void moe_sums(const MoeGemm& a, const MoeRows<NT>& ro
             q3_nibs(z.p[n].b[0], z.p[n].b[1], z.p[n].b[2], x);
             tr4(x[0], x[1], x[2], x[3], nib[n]);
         }
-        wave_lds_fence();
+        ti_wave_lds_fence();
         rows.load(z, st + W, G);
         load_x(st + W);
         TI_ISSUE_FENCE();

@@ -370,10 +370,12 @@ __global__ __launch_bounds__(64 * TA_W) void k_attn_tq8(TAttnArgs a) {
     };
 
     // ---- this wave's blocks of cached keys, the next block's loads in flight during the
-    // current one (LDS tile reuse is ordered: one wave's LDS accesses complete in order)
+    // current one
     int blk = gw;
     while (blk < nb) {
+        ti_wave_lds_fence();                             // the last block is read
         store_blk();
+        ti_wave_lds_fence();
         const int k0 = blk * TA_BLK;
         blk += NW;
         if (blk < nb) load_blk(blk * TA_BLK);

@@ -101,6 +101,7 @@ __global__ __launch_bounds__(256, 2) void k_tern_gemm(GemmMats m, const int8_t* 
     };
     float acc[NT][MT][4] = {};
     auto step = [&](const Step& s, int st) {
+        ti_wave_lds_fence();                       // the last step's reads are done
 #pragma unroll
         for (int q = 0; q < 4 * MT; q++) L.act[4 * q + j][r] = s.av[q];
 #pragma unroll
@@ -110,6 +111,7 @@ __global__ __launch_bounds__(256, 2) void k_tern_gemm(GemmMats m, const int8_t* 
         }
 #pragma unroll
         for (int t = 0; t < MT; t++) reinterpret_cast<int*>(L.xsum)[p4 * 16 * MT + 16 * t + l4] = -s.xs[t];
+        ti_wave_lds_fence();
         v4f sc[NT];
 #pragma unroll
         for (int n = 0; n < NT; n++) sc[n] = L.scale[16 * n + r];

@@ -230,6 +230,14 @@ __device__ __forceinline__ void ti_bf16x3(const float (&v)[8], ti_b8 (&op)[3]) {
     for (int i = 0; i < 3; i++) op[i] = __builtin_bit_cast(ti_b8, make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]));
 }
 
+// Between a wave's LDS writes and the reads of other lanes of the same wave, and between those reads and the
+// next writes: the LDS unit serves a wave in order, so there is nothing to wait for, but the compiler, which sees
+// one lane, may move either across the other where their addresses differ in that lane.
+__device__ __forceinline__ void ti_wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Keep every memory operation issued so far above this point: the scheduler may
 // otherwise sink a kernel's weight loads below the wait for its activation loads,
 // which serialises two memory round trips that were meant to overlap.
