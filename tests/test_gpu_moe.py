@@ -382,10 +382,13 @@ def test_moe_decode_rejects_bad_shapes(ctx):
 
 
 # ---- the fused T > 1 block ------------------------------------------------------------------
-@pytest.mark.parametrize("T,H,I,nE,topk", [(16, H, I, NE, TOPK), (3, H, I, NE, TOPK), (8, 4096, 1024, 8, 2),
-                                           (5, 1024, 4096, 100, 8)])
-def test_moe_prefill_fused_matches_chain(ctx, orc, T, H, I, nE, topk):
-    """ti_moe_prefill_q3 (5 launches) against the chain of separate calls it replaces
+# the last three: five and more pairs an expert, the matrix-core kernels; skewed: one expert in every token's choice,
+# one in none; 33 and 31 groups leave a remainder of the 4-group step
+@pytest.mark.parametrize("T,H,I,nE,topk,skew", [(16, H, I, NE, TOPK, False), (3, H, I, NE, TOPK, False), (8, 4096, 1024, 8, 2, False),
+                                                (5, 1024, 4096, 100, 8, False), (20, 1056, 992, 8, 2, False),
+                                                (50, 1056, 992, 8, 2, True), (128, H, I, NE, TOPK, False)])
+def test_moe_prefill_fused_matches_chain(ctx, orc, T, H, I, nE, topk, skew):
+    """ti_moe_prefill_q3 (5 launches, 4 from five pairs an expert) against the chain of separate calls it replaces
     (ti_router, ti_moe_gemm_q3 x 2, ti_swiglu, ti_moe_gemm_q3, ti_moe_combine): routing,
     gate/up, activations, expert outputs and the residual bit for bit; and the routing
     against the oracle's."""
@@ -396,6 +399,8 @@ def test_moe_prefill_fused_matches_chain(ctx, orc, T, H, I, nE, topk):
     normed = rng.standard_normal(T * H).astype(np.float32)
     logits = rng.standard_normal(T * nE).astype(np.float32)
     bias = (rng.standard_normal(nE) * 0.05).astype(np.float32)
+    if skew:
+        bias[1], bias[2] = 2.0, -2.0
     x = rng.standard_normal(T * H).astype(np.float32)
     d = {k: ctx.upload(v) for k, v in dict(normed=normed, logits=logits, bias=bias, p1=w1[0], s1=w1[1], p3=w3[0],
                                              s3=w3[1], p2=w2[0], s2=w2[1]).items()}
@@ -424,6 +429,8 @@ def test_moe_prefill_fused_matches_chain(ctx, orc, T, H, I, nE, topk):
         assert np.array_equal(runs[0][k].view(np.uint32), runs[1][k].view(np.uint32)), k
     oi, ow = orc.router(logits, bias, T, nE, topk)
     assert np.array_equal(runs[0]["idx"], oi)
+    if skew:
+        assert (oi == 1).sum() == T and (oi == 2).sum() == 0
     # the fused block against the oracle itself (models/lfm25.js:2145-2166), as
     # test_moe_block holds the chain: the expert activations first, then the block output
     # with the down projection teacher-forced on the GPU's activations (its int8
