@@ -16,10 +16,12 @@ def ctx():
 
 
 # K: one group, a remainder of the 4-group step, fewer steps than waves, whole rounds of them; N and T: one below,
-# at and above a 16-wide tile; between them every tile shape of the dispatch (the last two: 2 x 4 and 4 x 4 of 4 waves)
+# at and above a 16-wide tile; between them every tile shape of the dispatch at 256 CUs (the last five: 2 x 4 and
+# 4 x 4 of 4 waves, 1 x 2, 1 x 4 and 2 x 3 of 8)
 @pytest.mark.parametrize("T,N,K", [(2, 15, 32), (5, 17, 96), (16, 16, 160), (17, 33, 1120), (33, 4000, 288), (48, 4096, 64),
                                    (77, 2048, 2048), (95, 2064, 1056), (49, 4112, 320), (128, 4096, 128), (77, 6144, 96),
-                                   (256, 100, 3104), (5, 8000, 2016), (200, 6000, 256), (255, 9999, 64)])
+                                   (256, 100, 3104), (5, 8000, 2016), (200, 6000, 256), (255, 9999, 64), (31, 3000, 160),
+                                   (128, 2048, 1120), (47, 6100, 96)])
 def test_prompt_gemm_against_64_bits(ctx, orc, T, N, K):
     rng = np.random.default_rng(T * 7 + N + K)
     G = K // 32
