@@ -17,10 +17,11 @@ def ctx():
 
 
 # T x heads per KV head: one above the short kernel's 32 rows, around 64 and 128 rows, several workgroups; contexts from
-# the chunk alone to several ranges with a remainder. wide: V scales over six decades, a V above the f16 range
+# the chunk alone to several ranges with a remainder, and past 16384 keys, where 64 ranges grow. wide: V scales over six decades, a V above the f16 range
 @pytest.mark.parametrize("T,pos,nHq,nKv,wide", [(33, 0, 2, 2, False), (17, 62, 4, 2, True), (32, 64, 4, 2, False), (33, 31, 4, 2, True),
                                                 (65, 127, 2, 1, False), (11, 100, 12, 4, False), (64, 1000, 16, 4, True),
-                                                (256, 0, 2, 1, False), (100, 2777, 16, 8, True), (256, 1100, 8, 8, False)])
+                                                (256, 0, 2, 1, False), (100, 2777, 16, 8, True), (256, 1100, 8, 8, False),
+                                                (33, 17001, 2, 2, False)])
 def test_prompt_attention_against_64_bits(ctx, T, pos, nHq, nKv, wide):
     rng = np.random.default_rng(T + pos + nHq)
     S = pos + T
