@@ -298,14 +298,13 @@ __global__ __launch_bounds__(256) void k_quant_frag(const float* __restrict__ x,
 }
 
 // RMSNorm (the reference's 256 strided partials and tree, as k_rmsnorm) + quantQ8 -> fragments;
-// a workgroup per token. KU: H = 256 KU, every load issued before the first sum waits (2048 wide, 256
-// tokens: 6.0 -> 4.9 us); KU = 0: any H.
+// a workgroup per token. KU: H <= 256 KU, every load issued before the first sum waits (2048 wide, 256
+// tokens: 6.0 -> 4.9 us); KU = 0: any H. Elements past H are left out of their partial.
 template <int KU>
 __global__ __launch_bounds__(256) void k_norm_frag(const float* __restrict__ x, const uint16_t* __restrict__ nw, float eps,
-                                                   ti_h8* __restrict__ xh, float* __restrict__ xsc, int T, int Hany) {
+                                                   ti_h8* __restrict__ xh, float* __restrict__ xsc, int T, int H) {
     __shared__ float red[256];
     constexpr int NC = KU ? (KU + 7) / 8 : 1;              // 8-element chunks of a thread
-    const int H = KU ? 256 * KU : Hany;
     const int tok = blockIdx.x, G = H / 32, t = threadIdx.x;
     const size_t f0 = (size_t)(tok >> 4) * G;
     const int m = tok & 15;
@@ -323,7 +322,7 @@ __global__ __launch_bounds__(256) void k_norm_frag(const float* __restrict__ x, 
     if constexpr (KU > 0) {
         float xs[KU];
 #pragma unroll
-        for (int i = 0; i < KU; i++) xs[i] = xr[t + 256 * i];
+        for (int i = 0; i < KU; i++) xs[i] = xr[min(t + 256 * i, H - 1)];
 #pragma unroll
         for (int k = 0; k < NC; k++) load(k, min(t + 256 * k, H / 8 - 1));
         TI_ISSUE_FENCE();
@@ -331,7 +330,7 @@ __global__ __launch_bounds__(256) void k_norm_frag(const float* __restrict__ x, 
 #pragma unroll
         for (int i = 0; i < KU; i++) {
             const float sq = xs[i] * xs[i];
-            s = s + sq;
+            s = t + 256 * i < H ? s + sq : s;
         }
         float mean = ti_tree_sum_256(s, red) / (float)H;
         mean = mean + eps;
@@ -432,8 +431,9 @@ int ti_quant_frag_launch(ti_ctx* c, const float* x, const TiFrag& f, int T, int 
 int ti_norm_frag_launch(ti_ctx* c, const float* x, const uint16_t* w, float eps, const TiFrag& f, int T, int H) {
     const unsigned grid = (unsigned)((T + 15) / 16 * 16);
     ti_h8* xh = reinterpret_cast<ti_h8*>(f.xh);
-    if (H == 1024) k_norm_frag<4><<<grid, 256, 0, c->stream>>>(x, w, eps, xh, f.sc, T, H);
-    else if (H == 2048) k_norm_frag<8><<<grid, 256, 0, c->stream>>>(x, w, eps, xh, f.sc, T, H);
+    if (H <= 1024) k_norm_frag<4><<<grid, 256, 0, c->stream>>>(x, w, eps, xh, f.sc, T, H);
+    else if (H <= 2048) k_norm_frag<8><<<grid, 256, 0, c->stream>>>(x, w, eps, xh, f.sc, T, H);
+    else if (H <= 4096) k_norm_frag<16><<<grid, 256, 0, c->stream>>>(x, w, eps, xh, f.sc, T, H);
     else k_norm_frag<0><<<grid, 256, 0, c->stream>>>(x, w, eps, xh, f.sc, T, H);
     TI_LAUNCHED("k_norm_frag");
     return TI_OK;

@@ -100,10 +100,10 @@ def qwen_f64(cfg, W, kv, got, ids, P):
     return rows, int4_f64(W["lm_head.weight"], cfg["vocab"], d["H"]) @ rms(x[-1], f16("model.norm.weight"))
 
 
-# With 256 CUs the gate/up tile is 2, 4, 2 and 4 token tiles of 8 waves and 4 of 4 waves, the norm the 1024-wide,
-# 2048-wide and any-width one; the attention runs one and several key ranges, with and without a prefix
+# With 256 CUs the gate/up tile is 2, 4, 2 and 4 token tiles of 8 waves and 4 of 4 waves; the norm is run at and off the
+# widths its instances end at; the attention runs one and several key ranges, with and without a prefix
 @pytest.mark.parametrize("H,I,T,P", [(1024, 3072, 33, 5), (1024, 3072, 100, 0), (2048, 6144, 17, 70), (2048, 6144, 64, 0),
-                                     (2048, 6144, 256, 130), (512, 1056, 40, 700)])
+                                     (2048, 6144, 256, 130), (512, 1056, 40, 700), (256, 512, 20, 9), (3072, 512, 33, 0), (6144, 512, 18, 0)])
 def test_prompt_layer_against_64_bits(ctx, H, I, T, P):
     cfg = dict(layers=2, hidden=H, intermediate=I, n_heads=16, n_kv_heads=8, head_dim=HD, vocab=512, rope_theta=THETA,
                rms_eps=EPS, max_ctx=P + T, max_tokens=T)
