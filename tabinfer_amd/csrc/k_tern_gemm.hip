@@ -201,10 +201,11 @@ int ti_tern_gemm_mfma(ti_ctx* c, const int8_t* act, const int32_t* xsum, int K, 
     m.nmat = nmat;
     // Few tiles: one 16 x 16 tile a workgroup (its four waves split K), so that more CUs have
     // one; many: larger tiles, whose operands are read from LDS once for several products. us at
-    // 16 x 16, 32 x 16, 32 x 32 (rows x tokens): 2048 x 6144 x 50 (512 tiles) 7.0 / 7.4 / 10.2;
-    // 8192 x 2048 x 48 (1536) 6.9 / 5.9 / 6.6; 8192 x 6144 x 128 (4096) 36 / 28 / 24.5.
-    if (tiles < 1024) launch<1, 1>(c, m, act, xsum, K, B);
-    else if (tiles < 3072) launch<2, 1>(c, m, act, xsum, K, B);
+    // 16 x 16, 32 x 16, 32 x 32 (rows x tokens; 256 CUs): 2048 x 6144 x 50 (512 tiles) 7.0 / 7.4 / 10.2;
+    // 8192 x 2048 x 48 (1536) 6.9 / 5.9 / 6.6; 8192 x 6144 x 128 (4096) 36 / 28 / 24.5. The lines: four
+    // workgroups of the smallest tile a CU, and six of the next.
+    if (tiles < 4L * c->cus) launch<1, 1>(c, m, act, xsum, K, B);
+    else if (tiles < 12L * c->cus) launch<2, 1>(c, m, act, xsum, K, B);
     else launch<2, 2>(c, m, act, xsum, K, B);
     TI_LAUNCHED("k_tern_gemm");
     return TI_OK;
