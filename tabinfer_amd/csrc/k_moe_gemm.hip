@@ -15,8 +15,9 @@
 //
 // What bounds it at 16 pairs an expert is VALU work, 16 operations a (16 rows, group) to expand and
 // 8 a (16 rows, 16 pairs, group) to scale, beside the weights' way from HBM: the next step's weights are
-// in flight during one, and several workgroups share a CU. The block of 128 tokens x top-4 of 32
-// experts (2048 x 1792) takes 120 us, 75 + 38 of them here, against 186 with the kernel before (dot4
+// asked for at the start of one (loads return in order, so the wait for the second group's A operands, asked
+// for behind them, is a wait for them too), and three workgroups share a CU. The block of 128 tokens x
+// top-4 of 32 experts (2048 x 1792) takes 125 to 135 us (77 + 40 of them here in a trace), against 186 with the kernel before (dot4
 // in registers, a reduction over the lanes per pair).
 #include "ti_dev.h"
 #include "ti_moe.h"
@@ -202,7 +203,8 @@ __global__ __launch_bounds__(64 * W, 2) void k_moe_gemm(MoeGemm a) {
         rows.s[n] = (s ? a.s3[1] : a.s3[0]) + first;
         rows.off[n] = (uint32_t)min(16 * (GU ? n % 2 : n) + m, N - 1 - row0) * G;
     }
-    // the first routing ids before the weights, so that the scan waits for them alone
+    // the first routing ids before the weights (in the compiled code the scan's first wait is for both: the loop's
+    // later lists are asked for behind the weights)
     constexpr int NQ = SCAN / (64 * W);
     int rid[NQ];
     auto load_ids = [&](int c0) {

@@ -12,10 +12,11 @@
 //     f32's exponents, so a weight is as exact as in f32 beside any other, and what one key's scale is does not
 //     touch another's. (Two f16 under a common power of two take 5% less time, but lose all of a weight
 //     2^-36 of the largest scale of its keys.) The codes are exact in bf16.
-// What bounds it is latency first (a workgroup has 2 to 4 blocks; its loads of q are issued before all
-// else, and three workgroups share a CU), then the VALU work of the weights (scale, mask, exponential,
+// What bounds it is latency first (up to 16384 keys a workgroup has 2 to 4 blocks; its loads of q are issued
+// before all else, and three workgroups share a CU), then the VALU work of the weights (scale, mask, exponential,
 // four scaled three-fold splits). With 32 rows a wave, whose operands are read from LDS for two products, only two
-// fit: 256 tokens at 3840 47.7 against 46.7 us, at 0 26 against 15.
+// fit (with ranges of any length and weights in two halves, 256 tokens at 3840: 47.7 against 46.7 us, at 0: 26
+// against 15).
 // The ranges' partials (o, m, l; m in log2) are merged by k_pattn_merge, which also quantizes the output
 // into the o projection's fragments (k_gemm.hip) when asked.
 // 256 tokens x 16 heads over 4096 keys: 51.3 us with the merge, against 353 of k_attn_multi_q8 (P V as f32
@@ -369,14 +370,16 @@ int ti_pattn_launch(ti_ctx* c, const float* qr, const uint32_t* kq, const float*
     const int G = nHq / nKv, nrows = G * T, Smax = S0 + T - 1;
     const int nblk = (nrows + 63) / 64;
     const long kb = (Smax + KB - 1) / KB;
-    // key ranges: two workgroups a CU where there is work for them, else one, of at least two blocks (the merge reads
-    // every range's rows). us at one / two: 16 heads over 8, 256 tokens at 3840 54.0 / 46.7, at 1792 33.8 / 33.5,
-    // 64 at 4000 22.8 / 23.4, 100 at 1000 17.7 / 19.7, 20 at 6000 18.3 / 21.3
-    const long wg = (long)nKv * nblk, want = wg * kb >= 8L * c->cus ? 2L * c->cus : c->cus;
-    long ns = (want + wg - 1) / wg;
+    // key ranges: a workgroup a CU, of at least two blocks (the merge reads every range's rows). us at one a CU / two:
+    // 16 heads over 8, 256 tokens at 1792 34.1 / 34.1, 64 at 4000 23.7 / 23.0, 100 at 1000 18.7 / 19.3, 20 at 6000
+    // 19.0 / 21.6
+    const long wg = (long)nKv * nblk;
+    long ns = (c->cus + wg - 1) / wg;
     if (ns > (kb + 1) / 2) ns = (kb + 1) / 2;
-    // and of at most 256 keys: the output's running sum rounds twice per 32 keys (4096 keys in ranges of 512:
-    // error 2.7e-7 and 47.3 us, of 256: 2.3e-7 and 48.5)
+    // and, up to 16384 keys, of at most 256: the output's running sum rounds three times per 32 keys (256 tokens over
+    // 4096 keys in ranges of 512: error 2.7e-7 and 51.5 us, of 256: 2.4e-7 and 54.7; over 16256 in ranges of 2048: 4.7e-7,
+    // of 256: 2.7e-7). Past 16384 keys the merge's 64 ranges grow (32256 keys, ranges of 512: 3.2e-7; k_attn_multi_q8
+    // 4.6e-7)
     if (ns < (kb + 3) / 4) ns = (kb + 3) / 4;
     if (ns > 64) ns = 64;
     if (ns * T * nHq > TI_ATTN_ROWSPLITS) ns = TI_ATTN_ROWSPLITS / ((long)T * nHq);

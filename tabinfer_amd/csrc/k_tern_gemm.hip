@@ -12,7 +12,7 @@
 // block, codes 16j..16j+15 (the weights' 16 bytes shifted by 2j and masked) against the
 // activations' 16 bytes at 16j. In that layout neighbouring lanes are in different rows, and a
 // version that loaded its operands so from memory was bound by the scattered loads (14 us at
-// 2048 x 6144 x 50, 40 at 8192 x 6144 x 128; this one 7 and 25). So each wave loads whole 64- and
+// 2048 x 6144 x 50, 40 at 8192 x 6144 x 128; this one 6.4 and 26.7). So each wave loads whole 64- and
 // 256-byte runs, parks them in its own part of LDS and reads the operands from there; LDS
 // serves a wave in order, so there is no barrier in the loop.
 #include "ti_internal.h"
@@ -43,8 +43,10 @@ struct WaveBuf {
 };
 
 // Workgroup: a tile of 16 NT rows by 16 MT tokens (grid x: rows of the matrices in turn, y:
-// tokens); its 4 waves take every fourth step and their sums meet in LDS. Two steps of loads in
-// flight a wave.
+// tokens); its 4 waves take every fourth step and their sums meet in LDS. A wave holds two steps' registers, but
+// the compiler sinks the odd step's loads behind the test for the last step, to where they are used. Issued where
+// they are written (the odd step unconditional, issue fences) both steps are in flight and nothing is gained: 2048 x
+// 6144 x 50 6.4 us either way, 8192 x 6144 x 128 26.7 against 26.9.
 template <int NT, int MT>
 __global__ __launch_bounds__(256, 2) void k_tern_gemm(GemmMats m, const int8_t* __restrict__ act,
                                                       const int32_t* __restrict__ xsum, int K, int B) {
@@ -201,8 +203,8 @@ int ti_tern_gemm_mfma(ti_ctx* c, const int8_t* act, const int32_t* xsum, int K, 
     m.nmat = nmat;
     // Few tiles: one 16 x 16 tile a workgroup (its four waves split K), so that more CUs have
     // one; many: larger tiles, whose operands are read from LDS once for several products. us at
-    // 16 x 16, 32 x 16, 32 x 32 (rows x tokens; 256 CUs): 2048 x 6144 x 50 (512 tiles) 7.0 / 7.4 / 10.2;
-    // 8192 x 2048 x 48 (1536) 6.9 / 5.9 / 6.6; 8192 x 6144 x 128 (4096) 36 / 28 / 24.5. The lines: four
+    // 16 x 16, 32 x 16, 32 x 32 (rows x tokens; 256 CUs): 2048 x 6144 x 50 (512 tiles) 7.5 / 7.5 / 10.9;
+    // 8192 x 2048 x 48 (1536) 7.4 / 6.5 / 7.1; 8192 x 6144 x 128 (4096) 36.6 / 27.2 / 26.5. The lines: four
     // workgroups of the smallest tile a CU, and six of the next.
     if (tiles < 4L * c->cus) launch<1, 1>(c, m, act, xsum, K, B);
     else if (tiles < 12L * c->cus) launch<2, 1>(c, m, act, xsum, K, B);

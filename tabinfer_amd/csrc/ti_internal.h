@@ -125,7 +125,7 @@ int ti_tern_gemm_mfma(ti_ctx* c, const int8_t* act, const int32_t* xsum, int K, 
 int ti_tern_gemv_multi_norm(ti_ctx* c, const ti_tern_norm* nq, int K, int nmat, const uint8_t* const* codes,
                             const float* const* scales, float* const* outs, const int* Ns);
 // An activation [T][K] as the prompt GEMM reads it (k_gemm.hip): f16 codes [tile of 16 tokens]
-// [K / 32][64 lanes][8], and [tile][K / 32][32] floats: the tokens' scales, then -1032 * sum(codes)
+// [K / 32][64 lanes][8], and [tile][K / 32][16] floats, the tokens' scales
 struct TiFrag {
     uint32_t* xh;
     float* sc;
