@@ -241,7 +241,9 @@ int ti_tern_gemv_multi(ti_ctx* ctx, const int8_t* act, const int32_t* xsum, int 
                        const uint8_t* const* codes, const float* const* scales, float* const* outs,
                        const int* Ns);
 /* gemm_tern_b4 (cpu/kernel/src/lib.rs:331-367): B activation rows act[B*K], xsum[B*K/64];
- * row b of the output starts at out + b*out_stride. */
+ * row b of the output starts at out + b*out_stride. Up to 4 rows have ti_tern_gemv's bits each; more
+ * go through the matrix cores, which sum s*(dot - xsum) block by block: the same dots, f32 sums in
+ * another order and closer to 64 bits (2e-7 -> 5e-8), not the same bits. */
 int ti_tern_gemm(ti_ctx* ctx, float* out, long out_stride, const uint8_t* codes, const float* scales,
                  const int8_t* act, const int32_t* xsum, int N, int K, int B);
 /* quantize_act_into (tern.rs:206-222, mode 0) or WASM quantize (lib.rs:570-606,
@@ -319,7 +321,9 @@ int ti_bonsai_kv(ti_bonsai* m, int layer, float** kc, float** vc);   /* f32 [max
 int ti_bonsai_logits(ti_bonsai* m, float** logits);                   /* f32 [vocab], last decode */
 /* Model::forward per prompt token at positions pos.. (logits for the last one only, as n2's
  * prefill): history[pos..pos+T) = ids, argmax of the last logits -> history[pos+T], device
- * position = pos+T. ids == NULL takes the tokens already in the history. */
+ * position = pos+T. ids == NULL takes the tokens already in the history. Two and more tokens run as
+ * batches of up to 256 on the matrix cores (f32 sums in another order than a token's step, so not its
+ * bits); with a trace set, or one token, as steps. */
 int ti_bonsai_forward(ti_ctx* ctx, ti_bonsai* m, const int32_t* ids, int T, int pos);
 /* one token at the device position P: embeds history[P], writes KV row P, argmax ->
  * history[P+1], P += 1. Reads nothing from the host (capturable, replayable). */
@@ -375,7 +379,8 @@ int ti_moe_decode_q3(ti_ctx* ctx, float* x, const float* normed, const float* lo
  * router logits: router, moeGemm3 w1 and w3, swiglu, moeGemm3 w2, moeCombine) in five
  * launches instead of nine: the router shares a launch with normed's quantizer, normed is
  * quantized once for w1 and w3, both run in one launch,
- * and the SwiGLU is formed inside the quantizer of w2's input. The same arithmetic as that
+ * and the SwiGLU is formed inside the quantizer of w2's input; from five pairs an expert (T*topk >=
+ * 5*nE) in four, the SwiGLU and that quantizer inside w1 and w3's. The same arithmetic as that
  * chain of ti_router, ti_moe_gemm_q3, ti_swiglu, ti_moe_gemm_q3, ti_moe_combine: idx/wt[T*topk]
  * the routing, gate/up/act[T*topk*I] and out[T*topk*H] its intermediates, x[T*H] += the
  * combined experts. nE <= 256, H and I multiples of 32 <= 4096, T*H and T*topk*I <= 2^24;

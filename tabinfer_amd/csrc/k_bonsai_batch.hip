@@ -1,9 +1,9 @@
 // k_bonsai_batch.hip — the Bonsai decoder's kernels for a prompt's tokens together (T >= 2):
 // Model::forward per prompt token (native/crates/n2-core/src/model.rs:349-501, ops.rs), with
 // every per-token operation on T rows at once and the projections on the matrix cores
-// (k_tern_gemm.hip). Token by token a 48-token prompt through two layers took 3644 us (16
-// launches a token and every weight read 48 times); as one batch it takes
-// 159 us, 25 of them lm_head, the rest twenty-odd launches of 3-9 us.
+// (k_tern_gemm.hip). Token by token a 48-token prompt through two layers took 3610 us (16
+// launches a token and every weight read 48 times); as one batch it takes 157 us,
+// 26 of them lm_head, the rest 20 launches of 3-10 us and four around them.
 //
 // Rows are [token][width]. Widths are multiples of 1024; a row belongs to one workgroup of 256
 // threads, thread t holding elements 4 (t + 256 k) .. + 3.

@@ -798,9 +798,9 @@ __global__ void k_moe_combine(float* __restrict__ x, const float* __restrict__ o
 static inline bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // From five pairs an expert on the matrix cores win; below, their 16-pair tile is mostly padding and the
-// row kernels, which take a pair at a time, do less (block of 2048 x 1792, top-4 of 32 experts, us row kernels /
-// matrix cores: 2 pairs an expert 58 / 72, 4 75.7 / 78.2, 5 85.4 / 82.4, 16 186 / 120, 20 227 / 140; 512 x 512, 16 experts,
-// 25 pairs 73.9 / 32.6).
+// row kernels, which take a pair at a time, do less (block of 2048 x 1792, top-4 of 32 experts, the same inputs again, us
+// row kernels / matrix cores: 2 pairs an expert 58 / 74, 4 75.9 / 81.1, 5 85.8 / 82.5, 8 111 / 90.4, 16 186 / 120, 20 227 /
+// 140; 512 x 512, 16 experts, 25 pairs 94 / 40).
 static bool ti_moe_mfma(long P, int nE) { return P >= 5L * nE; }
 
 extern "C" int ti_requant43(ti_ctx* c, const uint32_t* pack4, const uint16_t* sc4, int rows, int K, uint32_t* p3,
