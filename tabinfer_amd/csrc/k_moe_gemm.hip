@@ -17,8 +17,9 @@
 // 8 a (16 rows, 16 pairs, group) to scale, beside the weights' way from HBM: the next step's weights are
 // asked for at the start of one (loads return in order, so the wait for the second group's A operands, asked
 // for behind them, is a wait for them too), and three workgroups share a CU. The block of 128 tokens x
-// top-4 of 32 experts (2048 x 1792) takes 125 to 135 us (77 + 40 of them here in a trace), against 186 with the kernel before (dot4
-// in registers, a reduction over the lanes per pair).
+// top-4 of 32 experts (2048 x 1792) takes 120 us on the same inputs again and 125 to 138 on others each time (78 + 41
+// of them here in a trace), against 186 to 190 with the kernel before (dot4 in registers, a reduction over the lanes
+// per pair).
 #include "ti_dev.h"
 #include "ti_moe.h"
 
